@@ -27,9 +27,9 @@ class OracleCounts(C.Structure):
 
 
 def build(reference: str = "/root/reference") -> None:
-    """make -C oracle (and the CImg harness when the reference tree exists)."""
+    """make -C oracle (and the CImg harness when the reference tree holds its vendored code)."""
     targets = ["all"]
-    if os.path.isdir(reference):
+    if os.path.isfile(os.path.join(reference, "vendor", "cimg", "CImg.h")):
         targets.append("ref")
     subprocess.run(["make", "-s", "-C", _HERE, f"REFERENCE={reference}"] + targets, check=True)
 
