@@ -40,11 +40,13 @@ hipError_t launch_text(uint8_t* frame, uint32_t W, uint32_t H, int32_t x0, int32
                        const uint8_t fg[3], const uint8_t bg[3], hipStream_t s);
 uint32_t raster_blocks_per_cu(int tile_size, bool fused, int mode, bool narrow, bool depth_in);
 hipError_t launch_copy(const void* src, void* dst, size_t n16, hipStream_t s);
-hipError_t launch_mlp_pack(const float* W, uint16_t* packed, hipStream_t s);
+hipError_t launch_mlp_pack(const float* W, uint16_t* packed, float* m, float* v, hipStream_t s);
 hipError_t launch_mlp_infer(const float* x, int64_t n, const uint16_t* packed, float* y, hipStream_t s);
 hipError_t launch_mlp_step(const float* samples, int64_t n, float* W, float* m, float* v, float* gpart,
-                           float* lpart, float* loss_out, int nblocks, uint64_t seed, uint32_t step, float lr,
+                           float* lpart, float* loss_out, int batch, uint64_t seed, uint32_t step, float lr,
                            float c1, float c2, hipStream_t s);
+int mlp_grad_parts(int batch);
+size_t mlp_grad_stride();
 }  // namespace rz
 
 using namespace rz;
@@ -2235,15 +2237,6 @@ rz_status mlp_buffers(rz_ctx* ctx) {
     return RZ_OK;
 }
 
-rz_status mlp_reset_adam(rz_ctx* ctx) {
-    std::vector<float> z(kMlpParams, 0.f);
-    RZ_HIP(ctx, hipMemcpyAsync(ctx->mlp_m.ptr, z.data(), kMlpParams * 4, hipMemcpyHostToDevice, ctx->stream));
-    RZ_HIP(ctx, hipMemcpyAsync(ctx->mlp_v.ptr, z.data(), kMlpParams * 4, hipMemcpyHostToDevice, ctx->stream));
-    RZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
-    ctx->mlp_steps = 0;
-    return RZ_OK;
-}
-
 }  // namespace
 
 rz_status rz_mlp_set_weights(rz_ctx* ctx, const float* params) {
@@ -2253,8 +2246,9 @@ rz_status rz_mlp_set_weights(rz_ctx* ctx, const float* params) {
     if (st != RZ_OK) return st;
     RZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
     RZ_HIP(ctx, hipMemcpy(ctx->mlp_w.ptr, params, kMlpParams * 4, hipMemcpyHostToDevice));
-    RZ_HIP(ctx, launch_mlp_pack((const float*)ctx->mlp_w.ptr, (uint16_t*)ctx->mlp_packed.ptr, ctx->stream));
-    if ((st = mlp_reset_adam(ctx)) != RZ_OK) return st;
+    RZ_HIP(ctx, launch_mlp_pack((const float*)ctx->mlp_w.ptr, (uint16_t*)ctx->mlp_packed.ptr, (float*)ctx->mlp_m.ptr,
+                                (float*)ctx->mlp_v.ptr, ctx->stream));
+    ctx->mlp_steps = 0;
     ctx->mlp_ready = true;
     return RZ_OK;
 }
@@ -2319,10 +2313,10 @@ rz_status rz_mlp_train(rz_ctx* ctx, const float* samples_device, int64_t n, int3
     if (!ctx || !samples_device || n <= 0 || steps < 1 || batch < 64) return RZ_ERR_INVALID_ARG;
     if (!ctx->mlp_ready) return fail(ctx, RZ_ERR_INVALID_ARG, "no network weights (rz_mlp_init first)");
     RZ_HIP(ctx, hipSetDevice(ctx->device));
-    const int nblocks = batch / 64;
+    const size_t parts = (size_t)mlp_grad_parts(batch);
     rz_status st;
-    if ((st = ensure(ctx, ctx->mlp_gpart, (size_t)nblocks * kMlpParams * 4)) != RZ_OK) return st;
-    if ((st = ensure(ctx, ctx->mlp_lpart, (size_t)nblocks * 4)) != RZ_OK) return st;
+    if ((st = ensure(ctx, ctx->mlp_gpart, parts * mlp_grad_stride() * 4)) != RZ_OK) return st;
+    if ((st = ensure(ctx, ctx->mlp_lpart, parts * 4)) != RZ_OK) return st;
     if ((st = ensure(ctx, ctx->mlp_loss, (size_t)steps * 4)) != RZ_OK) return st;
     for (int32_t k = 0; k < steps; ++k) {
         // cosine decay from lr to lr/100
@@ -2333,14 +2327,15 @@ rz_status rz_mlp_train(rz_ctx* ctx, const float* samples_device, int64_t n, int3
         const float c2 = 1.0f / (1.0f - std::pow(0.999f, (float)t));
         RZ_HIP(ctx, launch_mlp_step(samples_device, n, (float*)ctx->mlp_w.ptr, (float*)ctx->mlp_m.ptr,
                                     (float*)ctx->mlp_v.ptr, (float*)ctx->mlp_gpart.ptr, (float*)ctx->mlp_lpart.ptr,
-                                    (float*)ctx->mlp_loss.ptr + k, nblocks, seed, t, lr_k, c1, c2, ctx->stream));
+                                    (float*)ctx->mlp_loss.ptr + k, batch, seed, t, lr_k, c1, c2, ctx->stream));
     }
-    RZ_HIP(ctx, launch_mlp_pack((const float*)ctx->mlp_w.ptr, (uint16_t*)ctx->mlp_packed.ptr, ctx->stream));
+    RZ_HIP(ctx, launch_mlp_pack((const float*)ctx->mlp_w.ptr, (uint16_t*)ctx->mlp_packed.ptr, nullptr, nullptr,
+                                ctx->stream));
     if (losses)
         RZ_HIP(ctx, hipMemcpyAsync(losses, ctx->mlp_loss.ptr, (size_t)steps * 4, hipMemcpyDeviceToHost, ctx->stream));
     RZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
     if (losses)
-        for (int32_t k = 0; k < steps; ++k) losses[k] /= (float)(nblocks * 64);
+        for (int32_t k = 0; k < steps; ++k) losses[k] /= (float)(batch / 64 * 64);
     return RZ_OK;
 }
 

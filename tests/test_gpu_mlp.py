@@ -72,6 +72,45 @@ def test_one_training_step_matches_numpy_gradient(ctx):
     assert (np.abs(delta[zero]) <= 1e-6).mean() > 0.995
 
 
+def _drawn(n, batch, step, seed):
+    """The samples a training step draws: SplitMix64's mix of seed, step and place, modulo n."""
+    k = np.uint64(step * 1048576 + 1) + np.arange(batch, dtype=np.uint64)
+    with np.errstate(over="ignore"):
+        z = np.uint64(seed) + np.uint64(0x9E3779B97F4A7C15) * k
+        z = (z ^ (z >> np.uint64(30))) * np.uint64(0xBF58476D1CE4E5B9)
+        z = (z ^ (z >> np.uint64(27))) * np.uint64(0x94D049BB133111EB)
+        z = z ^ (z >> np.uint64(31))
+    return (z % np.uint64(n)).astype(np.int64)
+
+
+@pytest.mark.parametrize("n, batch", [(1, 64), (37, 64), (1000, 127), (5000, 64 * 256), (5000, 64 * 259)])
+def test_training_step_over_chunks(ctx, n, batch):
+    """One chunk of 64 samples, one per workgroup, and workgroups with a second chunk: the
+    step's loss and the sign of every gradient that is not tiny (the first Adam step is
+    -lr * sign(g)), against the numpy gradient over the same drawn samples."""
+    p = M.random_params(15, scale=0.5)
+    ctx.mlp_set_weights(p)
+    rng = np.random.default_rng(n)
+    data = np.concatenate([rng.uniform(-1, 1, (n, M.N_IN)), rng.uniform(0, 1, (n, M.N_OUT))], 1).astype(np.float32)
+    buf = ctx.empty(data.shape, np.float32)
+    lr = 1e-3
+    try:
+        buf.upload(data)
+        losses = ctx.mlp_train(buf, n, steps=1, batch=batch, lr=lr, seed=21)
+    finally:
+        buf.close()
+    rows = data[_drawn(n, batch // 64 * 64, 1, 21)]
+    loss, g = M.loss_and_grad(p, rows[:, :M.N_IN], rows[:, M.N_IN:])
+    assert abs(losses[0] - loss) <= 1e-4 * (1 + loss), (losses[0], loss)
+    delta = ctx.mlp_get_weights().astype(np.float64) - p.astype(np.float64)
+    # f32 sums of up to 16,576 terms, and a bf16 rounding of an activation falling the other
+    # way for one sample in some hundreds: well under 1e-3 of the largest gradient
+    big = np.abs(g) > 1e-3 * np.abs(g).max()
+    assert big.sum() > 1000
+    agree = np.abs(delta[big] + lr * np.sign(g[big])) <= 2e-3 * lr
+    assert agree.mean() > 0.995, agree.mean()
+
+
 def test_collect_train_and_shade(ctx):
     scene, args = scenes.learned_shading_scene(width=320, height=180, subdivisions=4, map_size=128)
     mesh = ctx.upload(scene)
