@@ -38,7 +38,7 @@ hipError_t launch_check_quotients(uint32_t blocks, uint32_t per_thread, uint32_t
                                   hipStream_t s);
 hipError_t launch_text(uint8_t* frame, uint32_t W, uint32_t H, int32_t x0, int32_t y0, const char* text,
                        const uint8_t fg[3], const uint8_t bg[3], hipStream_t s);
-uint32_t raster_blocks_per_cu(int tile_size, bool fused, int mode, bool narrow, bool depth_in);
+uint32_t raster_blocks_per_cu(int tile_size, bool fused, int mode, bool narrow, bool depth_in, bool drop);
 hipError_t launch_copy(const void* src, void* dst, size_t n16, hipStream_t s);
 hipError_t launch_mlp_pack(const float* W, uint16_t* packed, float* m, float* v, hipStream_t s);
 hipError_t launch_mlp_infer(const float* x, int64_t n, const uint16_t* packed, float* y, hipStream_t s);
@@ -91,6 +91,7 @@ struct rz_mesh {
     // from here and the bin pass gathers nothing (uniform = 1)
     int32_t uniform = 0, uniform_n = 0, uniform_t = -1, uniform_m = 0;
     float uniform_nrm[3] = {0.f, 0.f, 0.f};   // model-space normal uniform_n
+    bool overdrawn = false;                   // mesh_overdrawn
     DevMaterial* mats = nullptr;
     uint32_t* texels = nullptr;
     float* luts = nullptr;
@@ -483,6 +484,7 @@ void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args
     rp.ovf_list = bp.ovf_list;
     rp.front_mask = bp.front_mask;
     rp.face_v = mesh->bin_face_v;
+    rp.overdrawn = mesh->overdrawn ? 1 : 0;
     rp.max_blocks = lay.raster_grid;
     L.orp = rp;   // batches: k_overflow_batch
     L.orp.part_frag = part + lay.off_ovf;
@@ -548,13 +550,13 @@ int frame_bin_cap(const rz_ctx* ctx, const rz_mesh* mesh, uint32_t ntiles) {
 // in flight (1080p: 23 against 63 us; 4M triangles at 4096x4096: 326 against 254 us)
 // flags: the frame's; without RZ_FLAG_CLEARED the raster pass stages the input depths
 // in dynamic LDS, which the residency count includes.
-void frame_shape(const rz_ctx* ctx, const rz_args& a, int mode, uint32_t flags, uint32_t& ntiles, bool& narrow,
+void frame_shape(const rz_ctx* ctx, const rz_mesh* mesh, const rz_args& a, int mode, uint32_t flags, uint32_t& ntiles, bool& narrow,
                  uint32_t& grid) {
     ntiles = ((a.image_width + ctx->tile_size - 1) / ctx->tile_size) *
              ((a.image_height + ctx->tile_size - 1) / ctx->tile_size);
     narrow = ctx->tile_size == 16 && ntiles >= kNarrowTiles;
     const uint32_t per_cu =
-        raster_blocks_per_cu(ctx->tile_size, ctx->fused, mode, narrow, (flags & RZ_FLAG_CLEARED) == 0);
+        raster_blocks_per_cu(ctx->tile_size, ctx->fused, mode, narrow, (flags & RZ_FLAG_CLEARED) == 0, mesh->overdrawn);
     grid = (uint32_t)ctx->cus * per_cu / 8u * 8u;
     if (grid < 8) grid = 8;
 }
@@ -583,7 +585,7 @@ rz_status prepare_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
     if (mode < 0) mode = (flags & RZ_FLAG_MLP_SHADE) ? kShadeMlp : kShadePlain;
     uint32_t ntiles = 0, grid = 0;
     bool narrow = false;
-    frame_shape(ctx, *args, mode, flags, ntiles, narrow, grid);
+    frame_shape(ctx, mesh, *args, mode, flags, ntiles, narrow, grid);
     const int cap = frame_bin_cap(ctx, mesh, ntiles);
     const bool can_overflow = (uint32_t)cap < (uint32_t)mesh->nf;
     const FrameLayout lay = layout_frame(mesh, *args, ctx->tile_size, cap, ctx->fused, grid,
@@ -781,8 +783,8 @@ constexpr size_t kSyncWords = 3 * 8 * (kCountStride / 2);
 constexpr size_t kCursorWord = kSyncWords + 16;   // (64-bit words from the block's start)
 constexpr size_t kSyncBytes = (kCursorWord + 16) * 8;
 
-rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32_t flags, DevBuf& arena,
-                        DevBuf& tables, BatchLaunch& B) {
+rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32_t flags, bool stats,
+                        DevBuf& arena, DevBuf& tables, BatchLaunch& B) {
     if (n < 1 || !items) return fail(ctx, RZ_ERR_INVALID_ARG, "empty batch");
     if (n > kMaxBatchMeshes) return fail(ctx, RZ_ERR_INVALID_ARG, "batch of %d meshes: at most %d", n, kMaxBatchMeshes);
     if (!(flags & RZ_FLAG_DEVICE_BUFFERS))
@@ -843,6 +845,7 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
         fill_frame(it.mesh, it.lights, it.num_lights, it.args, flags, lays[i], ptrs, L);
         L.sp.mlp = (const uint16_t*)ctx->mlp_packed.ptr;
         bind_outputs(L, cleared, it.frame, it.depth, it.ids);
+        L.rp.count_frags = stats ? 1 : 0;
         // the shared lists; their 8 counters are the first mesh's (cleared by its vertex pass)
         const FrameLaunch& L0 = B.frames[0];
         L.bp.lists = lists;
@@ -931,8 +934,8 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
 // (two generations of counter lines), the tile lists and raster statistics shared, the
 // parameter tables holding each mesh's bin, raster and overflow parameters for generation 0
 // and then generation 1, and the barriers at the start of the arena, zeroed.
-rz_status prepare_batch_sync(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32_t flags, DevBuf& arena,
-                             DevBuf& tables, BatchLaunch& B) {
+rz_status prepare_batch_sync(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32_t flags, bool stats,
+                             DevBuf& arena, DevBuf& tables, BatchLaunch& B) {
     if (n < 1 || !items) return fail(ctx, RZ_ERR_INVALID_ARG, "empty batch");
     if (n > kMaxBatchMeshes) return fail(ctx, RZ_ERR_INVALID_ARG, "batch of %d meshes: at most %d", n, kMaxBatchMeshes);
     if (!(flags & RZ_FLAG_DEVICE_BUFFERS))
@@ -996,6 +999,7 @@ rz_status prepare_batch_sync(rz_ctx* ctx, const rz_batch_item* items, int32_t n,
             L.sp.mlp = (const uint16_t*)ctx->mlp_packed.ptr;
             L.sp.mode = B.mode;
             bind_outputs(L, cleared, it.frame, it.depth, it.ids);
+            L.rp.count_frags = stats ? 1 : 0;
             // the shared lists; their 8 counters, and the batch's overflow count, are the
             // first mesh's (its bin work zeroes the other generation's for the next frame)
             const FrameLaunch& L0 = g ? B.frames1[0] : B.frames[0];
@@ -1092,10 +1096,10 @@ rz_status prepare_batch_sync(rz_ctx* ctx, const rz_batch_item* items, int32_t n,
     return RZ_OK;
 }
 
-rz_status prepare_any_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32_t flags, DevBuf& arena,
-                            DevBuf& tables, BatchLaunch& B) {
-    return ctx->batch_persistent ? prepare_batch_sync(ctx, items, n, flags, arena, tables, B)
-                                 : prepare_batch(ctx, items, n, flags, arena, tables, B);
+rz_status prepare_any_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32_t flags, bool stats,
+                            DevBuf& arena, DevBuf& tables, BatchLaunch& B) {
+    return ctx->batch_persistent ? prepare_batch_sync(ctx, items, n, flags, stats, arena, tables, B)
+                                 : prepare_batch(ctx, items, n, flags, stats, arena, tables, B);
 }
 
 rz_status enqueue_batch(rz_ctx* ctx, const BatchLaunch& B, hipStream_t s, bool prof) {
@@ -1442,6 +1446,39 @@ void bin_faces(const rz_mesh_desc* d, std::vector<BinFace>& out) {
     }
 }
 
+// Whether a view of the mesh is likely to cover its pixels several times: the faces' total
+// area against the surface of the box their centroids spread over (model space), or against
+// its screen rectangle (raster space).  Seen from anywhere, front faces show about a quarter
+// of the area and the box a quarter of its surface, so the ratio is about the depth
+// complexity over the box: 0.5 for a sphere, tens for triangle soups.  (A side of the box:
+// the uniform distribution's 2 sqrt(3) standard deviations, which a few far vertices barely
+// move.)
+constexpr double kOverdrawn = 2.0;
+bool mesh_overdrawn(const rz_mesh_desc* d) {
+    const int stride = d->raster_space ? 4 : 3, dims = d->raster_space ? 2 : 3;
+    double area = 0.0, sum[3] = {0, 0, 0}, sq[3] = {0, 0, 0};
+    for (int32_t f = 0; f < d->num_faces; ++f) {
+        const float* v[3];
+        for (int k = 0; k < 3; ++k) v[k] = d->vertices + (size_t)stride * d->faces[f].vertices[k];
+        double e[3] = {0, 0, 0}, g[3] = {0, 0, 0};
+        for (int c = 0; c < dims; ++c) {
+            e[c] = (double)v[1][c] - v[0][c];
+            g[c] = (double)v[2][c] - v[0][c];
+            const double m = ((double)v[0][c] + v[1][c] + v[2][c]) / 3.0;
+            sum[c] += m;
+            sq[c] += m * m;
+        }
+        const double x = e[1] * g[2] - e[2] * g[1], y = e[2] * g[0] - e[0] * g[2], z = e[0] * g[1] - e[1] * g[0];
+        area += 0.5 * std::sqrt(x * x + y * y + z * z);
+    }
+    double side[3] = {0, 0, 0};
+    const double n = d->num_faces > 0 ? (double)d->num_faces : 1.0;
+    for (int c = 0; c < dims; ++c) side[c] = std::sqrt(12.0 * std::max(0.0, sq[c] / n - (sum[c] / n) * (sum[c] / n)));
+    const double box = d->raster_space ? side[0] * side[1]
+                                       : 2.0 * (side[0] * side[1] + side[1] * side[2] + side[2] * side[0]);
+    return area > kOverdrawn * box;   // (false for NaN)
+}
+
 }  // namespace
 
 rz_status rz_mesh_create(rz_ctx* ctx, const rz_mesh_desc* d, rz_mesh** out) {
@@ -1458,6 +1495,7 @@ rz_status rz_mesh_create(rz_ctx* ctx, const rz_mesh_desc* d, rz_mesh** out) {
     m->nf = d->num_faces;
     m->nm = d->num_materials;
     m->raster_space = d->raster_space != 0;
+    m->overdrawn = mesh_overdrawn(d);
     auto cleanup = [&](rz_status s) {
         rz_mesh_destroy(ctx, m);
         return s;
@@ -1781,6 +1819,7 @@ rz_status rz_draw_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
         }
     }
     bind_outputs(L, cleared, frame_d, depth_d, ids_d);
+    L.rp.count_frags = stats ? 1 : 0;
     if ((st = run_frame(ctx, L, ctx->profiling)) != RZ_OK) return st;
     if (!on_device) {
         RZ_HIP(ctx, hipMemcpyAsync(frame_buffer, frame_d, np * 3, hipMemcpyDeviceToHost, s));
@@ -2093,7 +2132,7 @@ void rz_graph_destroy(rz_graph* g) {
 rz_status rz_draw_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32_t flags, rz_frame_stats* stats) {
     if (!ctx) return RZ_ERR_INVALID_ARG;
     BatchLaunch B;
-    rz_status st = prepare_any_batch(ctx, items, n, flags, ctx->batch_arena, ctx->batch_tables, B);
+    rz_status st = prepare_any_batch(ctx, items, n, flags, stats != nullptr, ctx->batch_arena, ctx->batch_tables, B);
     if (st != RZ_OK) return st;
     const bool phase_clock = ctx->profiling && B.persistent;
     if (phase_clock) {
@@ -2153,7 +2192,7 @@ rz_status rz_batch_graph_create(rz_ctx* ctx, const rz_batch_item* items, int32_t
     gr->frames = frames;
     gr->owns_buffers = true;
     BatchLaunch B;
-    rz_status st = prepare_any_batch(ctx, items, n, flags, gr->arena, gr->tables, B);
+    rz_status st = prepare_any_batch(ctx, items, n, flags, false, gr->arena, gr->tables, B);
     if (st == RZ_OK)
         st = capture(ctx, frames, [&](int32_t, hipStream_t s) { return enqueue_batch(ctx, B, s, false); },
                      &gr->exec);
@@ -2180,7 +2219,7 @@ rz_status rz_autotune(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32
         ctx->tile_size = ts;
         ctx->bin_cap = 64;
         BatchLaunch B;
-        if ((st = prepare_any_batch(ctx, items, n, flags, ctx->batch_arena, ctx->batch_tables, B)) != RZ_OK) break;
+        if ((st = prepare_any_batch(ctx, items, n, flags, false, ctx->batch_arena, ctx->batch_tables, B)) != RZ_OK) break;
         if ((st = enqueue_batch(ctx, B, ctx->stream, false)) != RZ_OK) break;
         uint32_t need = 1;
         size_t tiles = 0;
@@ -2197,7 +2236,7 @@ rz_status rz_autotune(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32
         while (cap < need && cap < (1u << 20)) cap <<= 1;
         while (cap > 16 && tiles * (size_t)cap * 4 > kBinBudget) cap >>= 1;   // overflow path beyond the budget
         ctx->bin_cap = (int)cap;
-        if ((st = prepare_any_batch(ctx, items, n, flags, ctx->batch_arena, ctx->batch_tables, B)) != RZ_OK) break;
+        if ((st = prepare_any_batch(ctx, items, n, flags, false, ctx->batch_arena, ctx->batch_tables, B)) != RZ_OK) break;
         for (int w = 0; w < 3 && st == RZ_OK; ++w) st = enqueue_batch(ctx, B, ctx->stream, false);
         if (st != RZ_OK) break;
         const int reps = 10;
@@ -2365,7 +2404,7 @@ rz_status rz_draw_frame_noalloc(rz_ctx* ctx, const rz_mesh* mesh, rz_light* ligh
     RZ_HIP(ctx, hipSetDevice(ctx->device));
     uint32_t ntiles = 0, grid = 0;
     bool narrow = false;
-    frame_shape(ctx, *args, kShadePlain, flags, ntiles, narrow, grid);
+    frame_shape(ctx, mesh, *args, kShadePlain, flags, ntiles, narrow, grid);
     // Working set in `scratch`: the layout of rz_draw_frame with a bin capacity that fits.
     // With the fused pipeline and room for every face in every bin no tile can overflow
     // and the visibility buffer is never touched, so it takes no space.

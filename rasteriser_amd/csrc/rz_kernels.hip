@@ -76,6 +76,11 @@ __device__ __forceinline__ uint32_t wave_scan_incl(uint32_t v) {
     return (uint32_t)x;
 }
 
+// Set bits of a lane mask below this lane, added to n.
+__device__ __forceinline__ uint32_t bits_below(unsigned long long m, uint32_t n = 0u) {
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, n));
+}
+
 // Sum of v over the workgroup, stored by thread 0 (no atomics).  Every thread of the
 // workgroup must call it.
 __device__ __forceinline__ void store_block_sum(uint32_t v, uint32_t* out, int tid, int nthreads) {
@@ -875,6 +880,53 @@ __device__ __forceinline__ bool fragment_key_rcp(float pxf, float pyf, float x0,
     return key_from_edges(e0, e1, e2, z0, z1, z2, area, z);
 }
 
+// A lower bound (-inf: none) on the depth any pixel of the candidate rectangle
+// can get from the face.  The depth is z = (z0 b0 + z1 b1) + z2 b2 with every b_i >= 0, so
+// z >= zmin - |z|max (s + 4 u) where s bounds |b0 + b1 + b2 - 1| (u = 2^-24).  The exact
+// edge functions sum to the exact area at every point; each computed one is off by at most
+// 5.7 u L (D + 1) (shrink_rect), the computed area likewise with the vertices' own extent
+// for D, and the quotients add u each: s <= 8.55 u P (S + 2) / |area| + 2 u, with P the
+// perimeter (bounded by |dx| + |dy| sums) and S the larger of D and the extent.  12 for 8.55
+// covers the hardware reciprocal and the roundings of the bound; 8 u the other terms.
+// Slivers (s above 1/16), areas outside [2^-40, 2^40], infinite and NaN depths have none
+// (a NaN depth never passes the depth test).
+__device__ __forceinline__ float depth_floor(const float4& a, const float4& b, const float4& c, float X0, float X1,
+                                                float Y0, float Y1) {
+    const float vx0 = fminf(fminf(a.x, b.x), c.x), vx1 = fmaxf(fmaxf(a.x, b.x), c.x);
+    const float vy0 = fminf(fminf(a.y, b.y), c.y), vy1 = fmaxf(fmaxf(a.y, b.y), c.y);
+    const float D = fmaxf(fmaxf(vx1 - X0, X1 - vx0), fmaxf(vy1 - Y0, Y1 - vy0));
+    const float S = fmaxf(D, fmaxf(vx1 - vx0, vy1 - vy0));
+    const float P = ((fabsf(b.x - a.x) + fabsf(b.y - a.y)) + (fabsf(c.x - b.x) + fabsf(c.y - b.y))) +
+                    (fabsf(a.x - c.x) + fabsf(a.y - c.y));
+    const float area = fabsf(a.w);
+    const float e = (0x1.8p-21f * P) * (S + 2.0f) * __builtin_amdgcn_rcpf(area) + 0x1p-21f;
+    const float zmin = fminf(fminf(a.z, b.z), c.z), zabs = fmaxf(fmaxf(fabsf(a.z), fabsf(b.z)), fabsf(c.z));
+    const float z = zmin - zabs * e;
+    // (comparisons false for NaN)
+    const bool ok = (S <= 1048576.0f) & (area >= 0x1p-40f) & (area <= 0x1p40f) & (e <= 0.0625f) &
+                    (fabsf(z) <= 3.4028235e38f);
+    return ok ? z : -INFINITY;
+}
+
+// Buckets for a front-to-back order of depth bounds: by the bits of t = 1 - z (at least
+// 2^-24, the far plane), which the perspective depth spreads evenly over octaves of the eye
+// distance.  near: the largest bits among the bounds, whose buckets of 2^step follow; bucket
+// 0 holds the faces without a bound.
+__device__ __forceinline__ uint32_t bound_bits(float z) { return __float_as_uint(fmaxf(1.0f - z, 0x1p-24f)); }
+__device__ __forceinline__ int bucket_step(uint32_t near, uint32_t far) {
+    const uint32_t r = near - far;
+    return r < 64u ? 0 : 26 - __clz((int)r);
+}
+__device__ __forceinline__ uint32_t bound_bucket(float z, uint32_t near, int step) {
+    return z > -INFINITY ? min(63u, 1u + ((near - bound_bits(z)) >> step)) : 0u;
+}
+// depth_order of a value no bound of this bucket or a later one is below.  (1 - z rounds by
+// at most 2^-24 t, and exactly for z >= 1/2, where the edge's own rounding is monotone.)
+__device__ __forceinline__ uint32_t bucket_floor(uint32_t bucket, uint32_t near, int step) {
+    const float t = __uint_as_float(near - ((bucket - 1u) << step));
+    return bucket > 0u ? depth_order((1.0f - t) - t * 0x1p-22f) : 0u;
+}
+
 // One tile, by one workgroup.  The tile's bin is taken BLOCK faces at a time: the faces
 // whose bbox meets the tile are compacted (ballot + popcount ranks, wave totals in LDS)
 // and their counts of candidate pairs (two pixels of the face's rectangle in its tile)
@@ -883,6 +935,14 @@ __device__ __forceinline__ bool fragment_key_rcp(float pxf, float pyf, float x0,
 // found by counting the marks at or before it (per-word prefix counts + one popcount),
 // with no search.  A pair's two pixels share the face's LDS reads and the pixel's place
 // in the rectangle (a face with an odd count leaves one lane idle in its last pair).
+//
+// Overdraw: faces of a later chunk behind the tile's farthest pixel so far are dropped as
+// they are staged, and a chunk of kSortPairs or more is taken roughly front to back, so
+// that a pair whose face lies behind both its pixels is dropped before the edge functions
+// and a wave's remaining pairs once their faces lie behind the farthest pixel.  A face's depth bound is depth_floor's; 64 buckets between the chunk's nearest
+// and farthest bounds order the faces.  Dropped candidates could not have changed a key, so
+// the result is the same; only the count of inside-test fragments needs every one
+// (count_frags: a frame whose caller asked for statistics).
 //
 // FUSED: the workgroup then shades its own pixels from the LDS visibility words (the
 // deferred shade, without the round trip of the visibility buffer through HBM).  Tiles
@@ -904,24 +964,39 @@ __device__ __forceinline__ TileHead tile_head(const RasterParams& p, int tile, i
     return h;
 }
 
+// A tile of more faces than this may drop hidden candidates; a chunk of at least this many candidate pairs (eight candidates per pixel of the tile)
+// is taken front to back (raster_body).
+constexpr uint32_t kDropFaces = 32;
+template <int NPX>
+constexpr uint32_t kSortPairs = 4 * NPX;
+
 // Bytes of raster_body's scratch LDS: face data by rank, reused by the learned shader's
 // staging after the raster loop (and, in the batch-frame kernel, by its bin phase).
-template <int BLOCK, int MODE>
+template <int BLOCK, int MODE, bool DROP = true>
 struct RasterLds {
-    static constexpr int kRaster = 14 * BLOCK * 4;
+    static constexpr int kRaster = (DROP && BLOCK > 64 ? 15 : 14) * BLOCK * 4;
     static constexpr int kMlp = MODE == kShadeMlp ? (BLOCK / 64) * (64 * 16 * 2 + 64 * 4 * 4) : 0;
     static constexpr int kBytes = kRaster > kMlp ? kRaster : kMlp;
+};
+
+// What a workgroup does for its next tile while raster_body works on this one: ask() once
+// the first chunk is staged (no global read is awaited again before the next chunk or the
+// shading), entry() before the shading.  Single frames: nothing (their tiles are dealt
+// statically, walk_tiles).
+struct NoAhead {
+    __device__ __forceinline__ void ask() {}
+    __device__ __forceinline__ void entry() {}
 };
 
 // EXT_RAW: the scratch LDS (RasterLds bytes) is the caller's `raw`, else the function's own.
 // DYN_D0: the initial depths live in the launch's dynamic LDS (TS * TS floats when the
 // frame has an input depth buffer, none otherwise), not in a static array.
 template <int TS, int BLOCK, bool FUSED, int MODE, int SHRINK = kSlabPixels, bool EXT_RAW = false,
-          int SLAB = kSlabAlways, bool DYN_D0 = false>
+          int SLAB = kSlabAlways, bool DYN_D0 = false, bool DROP = true, typename Ahead = NoAhead>
 __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadeParams* sp, const float* s_lut,
                                             const DevMaterial* s_mats, const uint16_t* s_net, int tile,
                                             const TileHead& head, uint32_t& frags, uint32_t& cov,
-                                            unsigned char* raw = nullptr) {
+                                            unsigned char* raw = nullptr, Ahead ahead = Ahead()) {
     constexpr int NPX = TS * TS;
     constexpr int PPT = NPX / BLOCK;
     constexpr int NW = BLOCK / 64;
@@ -939,7 +1014,7 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
     }
     unsigned char* s_raw = raw;
     if constexpr (!EXT_RAW) {
-        __shared__ __align__(16) unsigned char s_own[RasterLds<BLOCK, MODE>::kBytes];
+        __shared__ __align__(16) unsigned char s_own[RasterLds<BLOCK, MODE, DROP>::kBytes];
         s_raw = s_own;
     }
     // x0 y0 z0 x1 y1 z1 x2 y2 z2 area refined_rcp(area)
@@ -947,8 +1022,11 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
     uint32_t* s_rect = reinterpret_cast<uint32_t*>(s_raw + 11 * BLOCK * 4);   // rx0 | ry0 << 8 | rw << 16
     uint32_t* s_face = s_rect + BLOCK;
     uint32_t* s_start = s_face + BLOCK;
+    uint32_t* s_zlow = s_start + BLOCK;        // depth_order of the depth bounds (early)
     __shared__ uint32_t s_wsum[NW], s_wlive[NW];
-    __shared__ unsigned long long s_mask[kWords];
+    // (two of each: a chunk resets the next one's)
+    __shared__ uint32_t s_hist[DROP && NW > 1 ? 2 : 1][DROP && NW > 1 ? 64 : 1], s_range[2][2];
+    __shared__ unsigned long long s_mask[kWords + 1];
     __shared__ uint32_t s_wpre[kWords];
 
     // an opaque copy of the thread index: values derived from it are recomputed for each
@@ -967,19 +1045,23 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
     // fills them: such a tile has no chunk and no stores here (uniform over the workgroup)
     const bool overflowed = count > p.cap;
     const uint32_t n = overflowed ? 0u : count;
+    const bool may_drop = DROP && n > (NW > 1 ? kDropFaces : (uint32_t)BLOCK) && !p.count_frags;   // (uniform)
     // the first chunk's face records, read before anything waits
-    float4 a0 = make_float4(0.f, 0.f, 0.f, 0.f), b0 = a0, c0 = a0;
+    uint32_t face = f_first;
+    float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a, c = a;
     if ((uint32_t)tid < n) {
-        const FaceRecord* r = p.rec + f_first;
-        a0 = r->r0; b0 = r->r1; c0 = r->r2;
+        const FaceRecord* r = p.rec + face;
+        a = r->r0; b = r->r1; c = r->r2;
     }
     // initial depths: the caller's depth buffer, staged in LDS, or 1 everywhere for a
     // frame without one (uniform; then nothing is staged)
     const bool has_d0 = p.depth_in != nullptr;
+    const bool whole = !DROP || ((uint32_t)ox + TS <= p.W && (uint32_t)oy + TS <= p.H);   // (uniform)
 #pragma unroll
     for (int j = 0; j < PPT; ++j) {
         const int l = tid + j * BLOCK;
-        s_key[l] = kEmptyKey;
+        // (a pixel outside the image holds the nearest key: never the tile's farthest)
+        s_key[l] = whole || (ox + (l % TS) < (int)p.W && oy + (l / TS) < (int)p.H) ? kEmptyKey : 0ull;
         if (has_d0) {
             const uint32_t x = ox + (l % TS), y = oy + (l / TS);
             float d0 = 1.0f;
@@ -987,27 +1069,44 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
             s_d0[l] = d0;
         }
     }
+    constexpr bool kSort = DROP && NW > 1;
+    if constexpr (kSort) {
+        if (tid < 64) s_hist[0][tid] = 0u;
+        if (tid < 2) s_range[0][tid] = tid ? ~0u : 0u;
+    }
     __syncthreads();
 
-    const unsigned long long below = (1ull << lane) - 1ull;
-    const unsigned long long upto = (below << 1) | 1ull;   // bits 0..lane
-    static_assert(BLOCK % 64 == 0, "candidates are dealt in whole waves");
-    // A chunk's faces (entry i of the bin: face f, record a b c) into the LDS face table
-    // by rank: their candidate rectangles, the prefix sums, the chunk's total of pairs.
-    struct Staged {
-        uint32_t cnt, start, total;
+    // the farthest depth a pixel of the tile holds, by every wave for itself
+    uint32_t zfar = ~0u;
+    auto read_zfar = [&]() {
+        uint32_t m = 0u;
+#pragma unroll
+        for (int j = 0; j < NPX / 64; ++j)
+            m = max(m, __hip_atomic_load(reinterpret_cast<uint32_t*>(s_key) + 2 * (lane + 64 * j) + 1, __ATOMIC_RELAXED,
+                                         __HIP_MEMORY_SCOPE_WORKGROUP));
+        zfar = (uint32_t)wave_reduce((int)m, 0, [](int x, int y) { return (int)max((uint32_t)x, (uint32_t)y); });
     };
-    auto stage = [&](uint32_t i, uint32_t f, const float4& a, const float4& b, const float4& c) -> Staged {
+
+    static_assert(BLOCK % 64 == 0, "candidates are dealt in whole waves");
+    int par = 0;
+    for (uint32_t base = 0; base < n; base += BLOCK, par ^= 1) {
+        // The chunk's faces (entry base + tid of the bin) into the LDS face table by rank:
+        // their candidate rectangles, the prefix sums, the chunk's total of pairs.
         uint32_t cnt = 0, rect = 0;
-        if (i < n) {
+        float zl = -INFINITY;
+        if (base + (uint32_t)tid < n) {
             const uint32_t lo = __float_as_uint(b.w), hi = __float_as_uint(c.w);
             int rx0 = max((int)(lo & 0xFFFFu) - ox, 0), rx1 = min((int)(hi & 0xFFFFu) - ox, TS - 1);
             int ry0 = max((int)(lo >> 16) - oy, 0), ry1 = min((int)(hi >> 16) - oy, TS - 1);
+            bool keep = rx0 <= rx1 && ry0 <= ry1;
+            if (may_drop && keep) {
+                zl = depth_floor(a, b, c, (float)(ox + rx0), (float)(ox + rx1), (float)(oy + ry0), (float)(oy + ry1));
+                keep = depth_order(zl) <= zfar;   // (else behind every pixel of the tile)
+            }
             // large rectangles: only the part the triangle can reach
-            bool keep = true;
-            if (rx0 <= rx1 && ry0 <= ry1 && (rx1 - rx0 + 1) * (ry1 - ry0 + 1) > SHRINK)
+            if (keep && (rx1 - rx0 + 1) * (ry1 - ry0 + 1) > SHRINK)
                 keep = shrink_rect<SLAB>(a, b, c, ox, oy, rx0, rx1, ry0, ry1);
-            if (keep && rx0 <= rx1 && ry0 <= ry1) {
+            if (keep) {
                 const uint32_t rw = rx1 - rx0 + 1, rh = ry1 - ry0 + 1;
                 cnt = (rw * rh + 1u) >> 1;   // candidate pairs
                 rect = (uint32_t)rx0 | ((uint32_t)ry0 << 8) | (rw << 16) | (rh << 24);
@@ -1032,44 +1131,60 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
                 if (w < wave) { wbase += sw; lbase += lw; }
                 total += sw;
             }
+            total = __builtin_amdgcn_readfirstlane(total);
         }
-        const uint32_t start = wbase + v - cnt;
+        uint32_t start = wbase + v - cnt, near = 0, bucket = 0;
+        int rank = (int)bits_below(live, lbase), step = 0;
+        const bool sorted = kSort && may_drop && total >= kSortPairs<NPX>;   // (uniform)
+        if (sorted) {
+            // Counting sort: one LDS atomic per face on its bucket's (faces << 20 | pairs)
+            // gives its place and first pair within the bucket, a wave scan of the 64 buckets
+            // the bucket's (at most 256 faces and 2^17 pairs).
+            auto mn = [](int x, int y) { return (int)min((uint32_t)x, (uint32_t)y); };
+            auto mx = [](int x, int y) { return (int)max((uint32_t)x, (uint32_t)y); };
+            const bool has = cnt > 0 && zl > -INFINITY;
+            const uint32_t h = (uint32_t)wave_reduce(has ? (int)bound_bits(zl) : 0, 0, mx);
+            const uint32_t l = (uint32_t)wave_reduce(has ? (int)bound_bits(zl) : -1, -1, mn);
+            if (lane == 0) {
+                atomicMax(&s_range[par][0], h);
+                atomicMin(&s_range[par][1], l);
+            }
+            __syncthreads();
+            near = __builtin_amdgcn_readfirstlane(s_range[par][0]);
+            step = near > 0 ? bucket_step(near, __builtin_amdgcn_readfirstlane(s_range[par][1])) : 0;
+            uint32_t at = 0;
+            if (cnt > 0) {
+                bucket = bound_bucket(zl, near, step);
+                at = atomicAdd(&s_hist[par][bucket], (1u << 20) | cnt);
+            }
+            __syncthreads();
+            const uint32_t hist = s_hist[par][lane];
+            const uint32_t hv = wave_scan_incl(hist);
+            at += (uint32_t)__shfl((int)(hv - hist), (int)bucket, 64);
+            rank = (int)(at >> 20);
+            start = at & 0xFFFFFu;
+        }
+        if constexpr (kSort) {
+            if (tid < 64) s_hist[par ^ 1][tid] = 0u;
+            if (tid < 2) s_range[par ^ 1][tid] = tid ? ~0u : 0u;
+        }
         if (cnt > 0) {
-            const int rank = (int)(lbase + (uint32_t)__popcll(live & below));
             s_v[0][rank] = a.x; s_v[1][rank] = a.y; s_v[2][rank] = a.z;
             s_v[3][rank] = b.x; s_v[4][rank] = b.y; s_v[5][rank] = b.z;
             s_v[6][rank] = c.x; s_v[7][rank] = c.y; s_v[8][rank] = c.z;
             s_v[9][rank] = a.w; s_v[10][rank] = refined_rcp(a.w);
             s_rect[rank] = rect;
-            s_face[rank] = f;
-            s_start[rank] = start;
+            s_face[rank] = face;
+            s_start[rank] = start | (bucket << 20);
+            if (sorted) s_zlow[rank] = depth_order(zl);
         }
-        return Staged{cnt, start, total};
-    };
-    // the first chunk from the records read above (which are then dead: they are not
-    // carried through the candidate loop), each later one read when its turn comes
-    Staged st{0u, 0u, 0u};
-    if (n > 0) st = stage((uint32_t)tid, f_first, a0, b0, c0);
-    for (uint32_t base = 0; base < n; base += BLOCK) {
-        if (base > 0) {
-            const uint32_t i = base + tid;
-            uint32_t f = 0;
-            float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a, c = a;
-            if (i < n) {
-                f = p.bins[(size_t)tile * p.cap + i];
-                const FaceRecord* r = p.rec + f;
-                a = r->r0; b = r->r1; c = r->r2;
-            }
-            st = stage(i, f, a, b, c);
-        }
-        const uint32_t cnt = st.cnt, start = st.start, total = st.total;
         // candidate pair k of face j (rank): the inside and depth tests of the pixels 2k and
         // 2k + 1 of its rectangle (row by row; the second only if the rectangle has it),
         // which share the face's reads and the pixel's place in the rectangle
-        auto test = [&](uint32_t k, int j) {
+        auto test = [&](bool early, uint32_t k, int j) {
             const uint32_t rc = s_rect[j];
             const uint32_t rw = (rc >> 16) & 0xFFu, rh = rc >> 24;
-            const uint32_t l = 2u * (k - s_start[j]);
+            const uint32_t l = 2u * (k - (s_start[j] & 0xFFFFFu));
             // l / rw exactly: |error| of the product < 1/(2*rw) for l < 1024
             const uint32_t dy = (uint32_t)(((float)l + 0.5f) * __builtin_amdgcn_rcpf((float)rw));
             const uint32_t dx = l - dy * rw;
@@ -1077,6 +1192,16 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
             const bool wrap = dx + 1u == rw;
             const int lx2 = wrap ? (int)(rc & 0xFFu) : lx + 1, ly2 = wrap ? ly + 1 : ly;
             const bool two = l + 1u < rw * rh;
+            if (early) {
+                // behind what both pixels hold already (a stale read is only farther)
+                const uint32_t zl = s_zlow[j];
+                const uint32_t* hi = reinterpret_cast<const uint32_t*>(s_key) + 1;
+                auto key_z = [&](int q) {
+                    return __hip_atomic_load(hi + 2 * q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                };
+                const uint32_t ka = key_z(ly * TS + lx), kb = two ? key_z(ly2 * TS + lx2) : 0u;
+                if (zl > max(ka, kb)) return;
+            }
             const float x0 = s_v[0][j], y0 = s_v[1][j], z0 = s_v[2][j], x1 = s_v[3][j], y1 = s_v[4][j];
             const float z1 = s_v[5][j], x2 = s_v[6][j], y2 = s_v[7][j], z2 = s_v[8][j], ar = s_v[9][j];
             const float ra = s_v[10][j];
@@ -1099,6 +1224,7 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
                 }
             }
         };
+        if (base == 0) ahead.ask();
         uint32_t before = 0;   // live faces whose first candidate precedes the round
         if constexpr (NW == 1) {
             // One wave: each pass of 64 candidate pairs finds their faces from a 64-bit mask of
@@ -1112,34 +1238,56 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
                 const uint32_t hi = wave_reduce(here && sb >= 32u ? (int)(1u << (sb - 32u)) : 0, 0, bor);
                 const unsigned long long m = ((unsigned long long)hi << 32) | lo;
                 const uint32_t k = r0 + (uint32_t)lane;
-                if (k < total) test(k, (int)(before + (uint32_t)__popcll(m & upto)) - 1);
+                // (the faces starting at or before the lane's pair: bits 0..lane of m)
+                if (k < total) test(false, k, (int)bits_below(m >> 1, before + (lo & 1u)) - 1);
                 before += (uint32_t)__popcll(m);
             }
         } else {
             for (uint32_t r0 = 0; r0 < total; r0 += kWords * 64) {
-                if (tid < kWords) s_mask[tid] = 0ull;
+                // a face's start s marks bit s - r0 + 63 of the words: pair k of the round (word
+                // w, lane l) counts the words up to w and the bits of word w + 1 below l
+                if (tid <= kWords) s_mask[tid] = 0ull;
                 __syncthreads();
                 if (cnt > 0 && start >= r0 && start - r0 < kWords * 64u)
-                    atomicOr(&s_mask[(start - r0) >> 6], 1ull << ((start - r0) & 63u));
+                    atomicOr(&s_mask[(start - r0 + 63u) >> 6], 1ull << ((start - r0 + 63u) & 63u));
                 __syncthreads();
-                if (wave == 0) {
-                    const uint32_t pc = (uint32_t)__popcll(s_mask[lane]);
-                    s_wpre[lane] = wave_scan_incl(pc) - pc;
-                }
+                if (wave == 0) s_wpre[lane] = wave_scan_incl((uint32_t)__popcll(s_mask[lane]));
                 __syncthreads();
                 const uint32_t r1 = min(total, r0 + kWords * 64u);
-                for (uint32_t k = r0 + tid; k < r1; k += BLOCK) {
-                    // (r0 and BLOCK are multiples of 64: candidate k's bit in its mask word
-                    // is the lane, so the mask of bits up to it is the loop-invariant upto)
-                    const uint32_t wi = (k - r0) >> 6;
-                    test(k, (int)(before + s_wpre[wi] + (uint32_t)__popcll(s_mask[wi] & upto)) - 1);
+                auto face_of = [&](uint32_t wi) { return (int)bits_below(s_mask[wi + 1], before + s_wpre[wi]) - 1; };
+                if constexpr (kSort) {
+                    uint32_t it = 0;
+                    for (uint32_t kw = r0 + 64u * (uint32_t)wave; kw < r1; kw += BLOCK, ++it) {   // (uniform over the wave)
+                        const uint32_t k = kw + (uint32_t)lane;
+                        const int j = face_of((kw - r0) >> 6);
+                        if (sorted && (it & 3u) == 3u) {
+                            // this face and all that follow behind the farthest pixel
+                            read_zfar();
+                            const uint32_t bucket = s_start[__builtin_amdgcn_readfirstlane(j)] >> 20;
+                            if (bucket_floor(bucket, near, step) > zfar) break;
+                        }
+                        if (k < r1) test(sorted, k, j);
+                    }
+                } else {
+                    for (uint32_t k = r0 + tid; k < r1; k += BLOCK) test(false, k, face_of((k - r0) >> 6));
                 }
-                before += s_wpre[kWords - 1] + (uint32_t)__popcll(s_mask[kWords - 1]);
+                before += s_wpre[kWords - 1] + (uint32_t)__popcll(s_mask[kWords]);
                 __syncthreads();   // the mask is cleared for the next round
             }
         }
         __syncthreads();       // ranks and wave totals are rewritten by the next chunk
+        // the next chunk's records, read here so that none are live through the candidates
+        const uint32_t i = base + BLOCK + (uint32_t)tid;
+        face = 0u;
+        a = b = c = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (i < n) {
+            face = p.bins[(size_t)tile * p.cap + i];
+            const FaceRecord* r = p.rec + face;
+            a = r->r0; b = r->r1; c = r->r2;
+        }
+        if (may_drop && base + BLOCK < n) read_zfar();
     }
+    ahead.entry();
     if (overflowed) return;
 
     if (FUSED && PPT > 1) {
@@ -1172,7 +1320,7 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
                 }
                 __syncthreads();   // s_wsum is rewritten by the next pass
             }
-            if (hit) s_hits[off + (uint32_t)__popcll(bal & below)] = (uint16_t)l;
+            if (hit) s_hits[bits_below(bal, off)] = (uint16_t)l;
             nh = tot;
         }
         __syncthreads();
@@ -1412,13 +1560,13 @@ __device__ __forceinline__ void walk_tiles(const RasterParams& p, const ListWalk
     }
 }
 
-template <int TS, int BLOCK>
+template <int TS, int BLOCK, bool DROP>
 __global__ __launch_bounds__(BLOCK, BLOCK == 256 ? 6 : 8) void k_raster(RasterParams p) {
     const ListWalk w(p);
     const bool overflow = overflowed_tiles(p);
     uint32_t frags = 0, cov = 0;
     walk_tiles(p, w, [&](int tile, const TileHead& h) {
-        raster_body<TS, BLOCK, false, kShadePlain, kSlabPixels, false, kSlabAlways, true>(
+        raster_body<TS, BLOCK, false, kShadePlain, kSlabPixels, false, kSlabAlways, true, DROP>(
             p, nullptr, nullptr, nullptr, nullptr, tile, h, frags, cov);
     });
     if (overflow)
@@ -1428,7 +1576,9 @@ __global__ __launch_bounds__(BLOCK, BLOCK == 256 ? 6 : 8) void k_raster(RasterPa
 // Raster and shade in one pass.
 // (the normalisation tables are read through the caches here: their LDS copy would cost
 // a resident workgroup per CU)
-template <int TS, int BLOCK, int MODE>
+// (DROP: the variant that drops hidden candidates; RasterParams::overdrawn says why it is
+// not the only one)
+template <int TS, int BLOCK, int MODE, bool DROP>
 __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 6) void k_raster_shade(RasterParams p, ShadeParams sp) {
     const float* s_lut = sp.luts;
     __shared__ __align__(16) uint16_t s_net[MODE == kShadeMlp ? kPackedBytes / 2 : 8];
@@ -1443,8 +1593,8 @@ __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 6) void k_raster_sha
     // (raster_body's first barrier orders these stores before any read)
     uint32_t frags = 0, cov = 0;
     walk_tiles(p, w, [&](int tile, const TileHead& h) {
-        raster_body<TS, BLOCK, true, MODE, kSlabPixels, false, kSlabAlways, true>(p, &sp, s_lut, s_mats, s_net,
-                                                                                  tile, h, frags, cov);
+        raster_body<TS, BLOCK, true, MODE, kSlabPixels, false, kSlabAlways, true, DROP>(p, &sp, s_lut, s_mats,
+                                                                                        s_net, tile, h, frags, cov);
     });
     if (overflow)
         frags += overflow_faces(p, blockIdx.x * BLOCK + threadIdx.x, gridDim.x * BLOCK);
@@ -1487,6 +1637,90 @@ __global__ __launch_bounds__(256) void k_shade(ShadeParams p) {
     }
 }
 
+// A batch's tiles differ in cost by orders of magnitude (overdraw), so workgroups take them
+// one at a time from per-list cursors (the second word of each list counter's line).  The
+// first tile needs no cursor: workgroup b has entry b / 8 of list b % 8, and the cursors
+// count from entry grid / 8 on.  The next take and its list entry are read while the
+// current tile is rasterised (TakeAhead); a workgroup whose list is empty looks at all
+// eight at once and takes from the next one with entries left.  (With a take before every
+// tile and one failed take per list at the end, a batch of 12 meshes and 7,000 tiles spent
+// most of its raster pass on cursors: every workgroup's chain of takes, each a device-wide
+// atomic on one of eight lines.)
+struct TakeAhead {
+    uint32_t* cursor;
+    const uint32_t* list;
+    uint32_t first, n;   // entries below `first` are dealt statically; the list's count
+    uint32_t* out;       // LDS: [0] the entry, [1] whether there is one (thread 0 writes)
+    uint32_t k = 0;
+    bool asked = false;
+    __device__ __forceinline__ void ask() {
+        asked = true;
+        if (threadIdx.x == 0) k = first + atomicAdd(cursor, 1u);
+    }
+    __device__ __forceinline__ void entry() {
+        if (!asked) ask();
+        if (threadIdx.x == 0) {
+            out[1] = k < n ? 1u : 0u;
+            if (k < n) out[0] = list[k];
+        }
+    }
+};
+
+// Calls body(entry, ahead) for every entry this workgroup takes; s_take: three LDS words.
+// Every thread calls it; the grid is a multiple of 8.
+template <typename Body>
+__device__ __forceinline__ void take_tiles(const BatchLists& bl, uint32_t* s_take, Body body) {
+    const uint32_t first = gridDim.x >> 3;
+    uint32_t x = blockIdx.x & 7u, k = blockIdx.x >> 3;
+    uint32_t n = bl.list_count[x * kCountStride];
+    bool have = k < n;   // (uniform)
+    uint32_t e = have ? bl.lists[(size_t)x * bl.stride + k] : 0u;
+    for (;;) {
+        if (!have) {
+            if (threadIdx.x < 64) {
+                const uint32_t y = (uint32_t)lane_id() & 7u;
+                uint32_t* line = bl.list_count + y * kCountStride;
+                const uint32_t c = __hip_atomic_load(line, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                const uint32_t u = __hip_atomic_load(line + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                uint32_t left = (uint32_t)(__ballot(first + u < c) & 0xFFull);   // (uniform)
+                uint32_t got = 0u, ge = 0u, gx = 0u;
+                while (left && !got) {
+                    // the first list at or after this workgroup's own, in turn
+                    const uint32_t own = blockIdx.x & 7u;
+                    const uint32_t rot = ((left >> own) | (left << (8u - own))) & 0xFFu;
+                    gx = (own + (uint32_t)__ffs((int)rot) - 1u) & 7u;
+                    left &= ~(1u << gx);
+                    uint32_t gk = 0u;
+                    if (threadIdx.x == 0) gk = first + atomicAdd(bl.list_count + gx * kCountStride + 1, 1u);
+                    gk = __builtin_amdgcn_readfirstlane(gk);
+                    if (gk < (uint32_t)__builtin_amdgcn_readlane((int)c, (int)gx)) {
+                        got = 1u;
+                        ge = bl.lists[(size_t)gx * bl.stride + gk];
+                    }
+                }
+                if (threadIdx.x == 0) {
+                    s_take[0] = ge;
+                    s_take[1] = got;
+                    s_take[2] = gx;
+                }
+            }
+            __syncthreads();
+            have = s_take[1] != 0u;
+            e = s_take[0];
+            x = __builtin_amdgcn_readfirstlane(s_take[2]);
+            if (!have) break;
+            n = bl.list_count[x * kCountStride];
+            __syncthreads();   // (s_take is rewritten for the next tile)
+        }
+        body(__builtin_amdgcn_readfirstlane(e),
+             TakeAhead{bl.list_count + x * kCountStride + 1, bl.lists + (size_t)x * bl.stride, first, n, s_take});
+        __syncthreads();
+        have = s_take[1] != 0u;
+        e = s_take[0];
+        __syncthreads();   // (s_take is rewritten for the next tile)
+    }
+}
+
 __global__ __launch_bounds__(256) void k_vertex_batch(const VertexParams* __restrict__ items,
                                                       const uint2* __restrict__ map) {
     const uint2 m = map[blockIdx.x];
@@ -1505,35 +1739,21 @@ __global__ __launch_bounds__(256) void k_bin_batch(const BinParams* __restrict__
 }
 // A batch's raster pass: one resident grid over the tile lists the meshes share, entry
 // (mesh << kListMeshShift) | tile, raster and shade of the tile with its mesh's
-// parameters.  A batch's tiles differ in cost by orders of magnitude (overdraw), so
-// workgroups take tiles one at a time from per-list cursors (the second word of each
-// list counter's line): first list b % 8, then the others in turn.  Every cursor only
-// grows, so each workgroup leaves after one failed take per list.
+// parameters.
 template <int TS, int BLOCK, int MODE>
 __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 6) void k_raster_shade_batch(
     const RasterParams* __restrict__ items, const ShadeParams* __restrict__ sitems, BatchLists bl) {
     __shared__ __align__(16) uint16_t s_net[MODE == kShadeMlp ? kPackedBytes / 2 : 8];
-    __shared__ uint32_t s_take;
+    __shared__ uint32_t s_take[3];
     if (MODE == kShadeMlp) stage_net(sitems[0].mlp, s_net, threadIdx.x, BLOCK);   // one network per batch
     uint32_t frags = 0, cov = 0;
-    for (uint32_t j = 0; j < 8; ++j) {
-        const uint32_t x = (blockIdx.x + j) & 7u;
-        const uint32_t n = bl.list_count[x * kCountStride];
-        uint32_t* cursor = bl.list_count + x * kCountStride + 1;
-        for (;;) {
-            if (threadIdx.x == 0) s_take = atomicAdd(cursor, 1u);
-            __syncthreads();
-            const uint32_t k = s_take;
-            __syncthreads();   // (s_take is rewritten by the next take)
-            if (k >= n) break;
-            const uint32_t e = bl.lists[(size_t)x * bl.stride + k];
-            const uint32_t m = e >> kListMeshShift;
-            const int tile = (int)(e & kListTileMask);
-            raster_body<TS, BLOCK, true, MODE, kShrinkPixels, false, kSlabAlways>(
-                items[m], &sitems[m], sitems[m].luts, nullptr, s_net, tile, tile_head(items[m], tile, threadIdx.x),
-                frags, cov);
-        }
-    }
+    take_tiles(bl, s_take, [&](uint32_t e, TakeAhead ahead) {
+        const uint32_t m = e >> kListMeshShift;
+        const int tile = (int)(e & kListTileMask);
+        raster_body<TS, BLOCK, true, MODE, kShrinkPixels, false, kSlabAlways>(
+            items[m], &sitems[m], sitems[m].luts, nullptr, s_net, tile, tile_head(items[m], tile, threadIdx.x), frags,
+            cov, nullptr, ahead);
+    });
     __syncthreads();
     store_block_sum(frags, bl.part_frag + blockIdx.x, threadIdx.x, BLOCK);
     store_block_sum(cov, bl.part_cov + blockIdx.x, threadIdx.x, BLOCK);
@@ -1628,7 +1848,7 @@ __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 4) void k_batch_fram
     __shared__ __align__(16) unsigned char s_lds[BatchFrameLds<BLOCK, MODE>::kBytes];
     __shared__ __align__(16) uint16_t s_net[MODE == kShadeMlp ? kPackedBytes / 2 : 8];
     __shared__ unsigned long long s_frame;
-    __shared__ uint32_t s_take;
+    __shared__ uint32_t s_take[3];
     if (MODE == kShadeMlp) stage_net(sitems[0].mlp, s_net, threadIdx.x, BLOCK);   // one network per batch
     // this frame's number: every workgroup of the previous frames has arrived at barrier 2
     if (threadIdx.x == 0) {
@@ -1653,9 +1873,9 @@ __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 4) void k_batch_fram
     // item's first wait for its own loads then also waits for the atomic; 3.74, 4.00 and
     // 4.29 ms taking 2, 4 or 8 consecutive items).
     phase_clock(q, 0, true);
-    if (threadIdx.x == 0) s_take = atomicAdd(q.cursor, 1u);
+    if (threadIdx.x == 0) s_take[0] = atomicAdd(q.cursor, 1u);
     __syncthreads();
-    uint32_t i = s_take;
+    uint32_t i = s_take[0];
     __syncthreads();   // (s_take is rewritten below)
     while (i < q.nB) {
         const uint2 m = q.bmap[i];
@@ -1669,9 +1889,9 @@ __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 4) void k_batch_fram
         else
             clear_body<BLOCK>(p, m.y - nb - nz, p.clear_blocks);
         __syncthreads();   // (s_lds is reused by the next item)
-        if (threadIdx.x == 0) s_take = atomicAdd(q.cursor, 1u);
+        if (threadIdx.x == 0) s_take[0] = atomicAdd(q.cursor, 1u);
         __syncthreads();
-        i = s_take;
+        i = s_take[0];
         __syncthreads();
     }
     phase_clock(q, 0, false);
@@ -1679,28 +1899,16 @@ __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 4) void k_batch_fram
     // every take of this frame is done: the cursor starts the next frame at zero
     if (w == 0 && threadIdx.x == 0) __hip_atomic_store(q.cursor, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 
-    // phase 2: tiles of the shared lists, one at a time from per-list cursors (first list
-    // w % 8, then the others)
+    // phase 2: tiles of the shared lists (take_tiles)
     uint32_t frags = 0, cov = 0, cov_ovf = 0;
     phase_clock(q, 1, true);
-    for (uint32_t j = 0; j < 8; ++j) {
-        const uint32_t x = (w + j) & 7u;
-        const uint32_t n = bl.list_count[x * kCountStride];
-        uint32_t* cursor = bl.list_count + x * kCountStride + 1;
-        for (;;) {
-            if (threadIdx.x == 0) s_take = atomicAdd(cursor, 1u);
-            __syncthreads();
-            const uint32_t k = s_take;
-            __syncthreads();   // (s_take is rewritten by the next take)
-            if (k >= n) break;
-            const uint32_t e = bl.lists[(size_t)x * bl.stride + k];
-            const uint32_t m = e >> kListMeshShift;
-            const int tile = (int)(e & kListTileMask);
-            raster_body<TS, BLOCK, true, MODE, kShrinkPixels, true, kSlabAlways>(
-                ritems[gen * nm + m], &sitems[m], sitems[m].luts, nullptr, s_net, tile,
-                tile_head(ritems[gen * nm + m], tile, threadIdx.x), frags, cov, s_lds);
-        }
-    }
+    take_tiles(bl, s_take, [&](uint32_t e, TakeAhead ahead) {
+        const uint32_t m = e >> kListMeshShift;
+        const int tile = (int)(e & kListTileMask);
+        raster_body<TS, BLOCK, true, MODE, kShrinkPixels, true, kSlabAlways>(
+            ritems[gen * nm + m], &sitems[m], sitems[m].luts, nullptr, s_net, tile,
+            tile_head(ritems[gen * nm + m], tile, threadIdx.x), frags, cov, s_lds, ahead);
+    });
     phase_clock(q, 1, false);
 
     // phases 3 and 4, when a bin overflowed (uniform: the count is final after barrier 0)
@@ -1961,32 +2169,40 @@ hipError_t launch_bin(const BinParams& p, hipStream_t s) {
 
 // Resident workgroups per CU of the list-driven raster kernel for this configuration.
 // depth_in: the frame stages an input depth buffer (the kernels' dynamic LDS).
-uint32_t raster_blocks_per_cu(int tile_size, bool fused, int mode, bool narrow, bool depth_in) {
+// drop: the mesh is overdrawn.
+uint32_t raster_blocks_per_cu(int tile_size, bool fused, int mode, bool narrow, bool depth_in, bool drop) {
     const void* f = nullptr;
     int block = 256;
-#define RZ_PICK(TS, B)                                                                              \
+#define RZ_PICK(TS, B, DROP)                                                                        \
     block = B;                                                                                      \
     if (!fused)                                                                                     \
-        f = reinterpret_cast<const void*>(&k_raster<TS, B>);                                         \
+        f = reinterpret_cast<const void*>(&k_raster<TS, B, DROP>);                                   \
     else if (mode == kShadeMlp)                                                                     \
-        f = reinterpret_cast<const void*>(&k_raster_shade<TS, B, kShadeMlp>);                        \
+        f = reinterpret_cast<const void*>(&k_raster_shade<TS, B, kShadeMlp, DROP>);                  \
     else if (mode == kShadeCollect)                                                                 \
-        f = reinterpret_cast<const void*>(&k_raster_shade<TS, B, kShadeCollect>);                    \
+        f = reinterpret_cast<const void*>(&k_raster_shade<TS, B, kShadeCollect, DROP>);              \
     else if (mode == kShadeChain)                                                                   \
-        f = reinterpret_cast<const void*>(&k_raster_shade<TS, B, kShadeChain>);                      \
+        f = reinterpret_cast<const void*>(&k_raster_shade<TS, B, kShadeChain, DROP>);                \
     else                                                                                            \
-        f = reinterpret_cast<const void*>(&k_raster_shade<TS, B, kShadePlain>);
+        f = reinterpret_cast<const void*>(&k_raster_shade<TS, B, kShadePlain, DROP>);
+#define RZ_PICK2(TS, B)          \
+    if (drop) {                  \
+        RZ_PICK(TS, B, true)     \
+    } else {                     \
+        RZ_PICK(TS, B, false)    \
+    }
     switch (tile_size) {
-        case 8: RZ_PICK(8, 64) break;
+        case 8: RZ_PICK2(8, 64) break;
         case 16:
             if (narrow) {
-                RZ_PICK(16, 64)
+                RZ_PICK2(16, 64)
             } else {
-                RZ_PICK(16, 256)
+                RZ_PICK2(16, 256)
             }
             break;
-        default: RZ_PICK(32, 256) break;
+        default: RZ_PICK2(32, 256) break;
     }
+#undef RZ_PICK2
 #undef RZ_PICK
     // (the walk over the tile lists is a static stride: a workgroup beyond residency
     // starts its tiles only when another workgroup ends, doubling the launch's tail)
@@ -2005,46 +2221,54 @@ __host__ __forceinline__ size_t d0_lds_bytes(const RasterParams& p, int tile_siz
 }
 
 hipError_t launch_raster(const RasterParams& p, int tile_size, hipStream_t s) {
-    const uint32_t grid = p.max_blocks;
     const size_t dyn = d0_lds_bytes(p, tile_size);
+#define RZ_LAUNCH(TS, B, DROP) hipLaunchKernelGGL((k_raster<TS, B, DROP>), dim3(p.max_blocks), dim3(B), dyn, s, p)
+#define RZ_LAUNCH2(TS, B)               \
+    if (p.overdrawn)                    \
+        RZ_LAUNCH(TS, B, true);         \
+    else                                \
+        RZ_LAUNCH(TS, B, false)
     switch (tile_size) {
-        case 8: hipLaunchKernelGGL((k_raster<8, 64>), dim3(grid), dim3(64), dyn, s, p); break;
+        case 8: RZ_LAUNCH2(8, 64); break;
         case 16:
-            if (p.narrow)
-                hipLaunchKernelGGL((k_raster<16, 64>), dim3(grid), dim3(64), dyn, s, p);
-            else
-                hipLaunchKernelGGL((k_raster<16, 256>), dim3(grid), dim3(256), dyn, s, p);
+            if (p.narrow) {
+                RZ_LAUNCH2(16, 64);
+            } else {
+                RZ_LAUNCH2(16, 256);
+            }
             break;
-        case 32: hipLaunchKernelGGL((k_raster<32, 256>), dim3(grid), dim3(256), dyn, s, p); break;
+        case 32: RZ_LAUNCH2(32, 256); break;
         default: return hipErrorInvalidValue;
     }
+#undef RZ_LAUNCH2
+#undef RZ_LAUNCH
     return hipGetLastError();
 }
 
 template <int MODE>
 hipError_t launch_raster_shade_mode(const RasterParams& p, const ShadeParams& sp, int tile_size, hipStream_t s) {
     const size_t dyn = d0_lds_bytes(p, tile_size);
+#define RZ_LAUNCH(TS, B, DROP) \
+    hipLaunchKernelGGL((k_raster_shade<TS, B, MODE, DROP>), dim3(p.max_blocks), dim3(B), dyn, s, p, sp)
+#define RZ_LAUNCH2(TS, B)               \
+    if (p.overdrawn)                    \
+        RZ_LAUNCH(TS, B, true);         \
+    else                                \
+        RZ_LAUNCH(TS, B, false)
     switch (tile_size) {
-        case 8: {
-            const uint32_t grid = p.max_blocks;
-            hipLaunchKernelGGL((k_raster_shade<8, 64, MODE>), dim3(grid), dim3(64), dyn, s, p, sp);
+        case 8: RZ_LAUNCH2(8, 64); break;
+        case 16:
+            if (p.narrow) {
+                RZ_LAUNCH2(16, 64);
+            } else {
+                RZ_LAUNCH2(16, 256);
+            }
             break;
-        }
-        case 16: {
-            const uint32_t grid = p.max_blocks;
-            if (p.narrow)
-                hipLaunchKernelGGL((k_raster_shade<16, 64, MODE>), dim3(grid), dim3(64), dyn, s, p, sp);
-            else
-                hipLaunchKernelGGL((k_raster_shade<16, 256, MODE>), dim3(grid), dim3(256), dyn, s, p, sp);
-            break;
-        }
-        case 32: {
-            const uint32_t grid = p.max_blocks;
-            hipLaunchKernelGGL((k_raster_shade<32, 256, MODE>), dim3(grid), dim3(256), dyn, s, p, sp);
-            break;
-        }
+        case 32: RZ_LAUNCH2(32, 256); break;
         default: return hipErrorInvalidValue;
     }
+#undef RZ_LAUNCH2
+#undef RZ_LAUNCH
     return hipGetLastError();
 }
 

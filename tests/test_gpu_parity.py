@@ -3,7 +3,8 @@ the same seeded inputs.  Face ids, depth bits and colour bytes must match exactl
 import numpy as np
 import pytest
 
-from rasteriser_amd import scenes
+import oracle
+from rasteriser_amd import MaterialSpec, Scene, make_args, make_faces, make_lights, scenes
 from tests.parity import check
 
 pytestmark = pytest.mark.gpu
@@ -49,6 +50,108 @@ def test_large_triangles_and_slivers(ctx, tile, cap):
     scene, args = scenes.large_triangle_scene(n=600)
     gpu, ref = check(ctx, scene, args, tuning=(tile, cap), label=f"large triangles tile {tile}")
     assert ref[3]["fragments"] > 5_000_000
+
+
+def overdraw_scene(n, W, H, seed):
+    """n screen-space triangles of 3-120 px over a small image: a third flat at one of a few
+    depths (ties between faces, -0 and 0, the depth a cleared pixel holds), a third steep,
+    a third slivers; some with infinite or NaN depths; half wound backwards."""
+    rng = np.random.default_rng(seed)
+    c = rng.uniform(0, 1, (n, 1, 2)) * [W, H]
+    ang = rng.uniform(0, 2 * np.pi, (n, 1)) + np.array([[0.0, 2.1, 4.2]])
+    rad = np.exp(rng.uniform(np.log(3), np.log(120), (n, 1)))
+    xy = c + rad[:, :, None] * np.stack([np.cos(ang), -np.sin(ang)], 2)
+    kind = rng.integers(0, 3, n)
+    sl = kind == 2
+    xy[sl, 2] = xy[sl, 0] + (xy[sl, 1] - xy[sl, 0]) * 0.4 + rng.uniform(-0.5, 0.5, (sl.sum(), 2))
+    z = rng.uniform(-1, 1, (n, 3))
+    z[kind == 0] = rng.choice([-0.0, 0.0, -0.5, 0.25, 0.25 + 2.0 ** -24, 1.0], ((kind == 0).sum(), 1))
+    bad = rng.random(n) < 0.02
+    z[bad, rng.integers(0, 3, bad.sum())] = rng.choice([np.inf, -np.inf, np.nan], bad.sum())
+    verts = np.concatenate([xy, z[:, :, None], np.ones((n, 3, 1))], 2).reshape(-1, 4).astype(np.float32)
+    tri = np.arange(3 * n).reshape(n, 3)
+    back = rng.random(n) < 0.5
+    tri[back] = tri[back][:, [0, 2, 1]]
+    scene = Scene(verts, np.array([[0.0, 0.0, 1.0]], np.float32), np.zeros((1, 2), np.float32),
+                  make_faces(tri, n=np.zeros_like(tri), t=None), [MaterialSpec((0.9, 0.8, 0.7))],
+                  make_lights([[0.0, 0.0, -1.0]], [200.0 * np.pi], [[1.0, 0.9, 0.8]]), raster_space=True)
+    return scene, make_args(W, H)
+
+
+def _draw_plain(ctx, mesh, scene, args, depth, fused=True, tuning=(16, 0)):
+    """A frame drawn without statistics (the raster pass then drops hidden candidates)."""
+    ctx.set_tuning(*tuning)
+    ctx.set_fused_shade(fused)
+    try:
+        f = None if depth is None else np.full((3, args.image_height, args.image_width), 7, np.uint8)
+        return ctx.draw(mesh, scene.lights_copy(), args, frame=f, depth=None if depth is None else depth.copy(),
+                        ids=True)[:3]
+    finally:
+        ctx.set_tuning(16, 0)
+        ctx.set_fused_shade(True)
+
+
+def _assert_frame(got, ref, label):
+    for name, a, b in zip(("face ids", "depth", "colour"), (got[2], got[1].view(np.uint32), got[0]),
+                          (ref[2], ref[1].view(np.uint32), ref[0])):
+        bad = np.argwhere(a != b)
+        assert bad.size == 0, f"{label}: {len(bad)} {name} differ, first at {bad[:3].tolist()}"
+
+
+@pytest.mark.parametrize("tuning", [(16, 0), (8, 0), (32, 0), (16, 300)])
+@pytest.mark.parametrize("n,W,H", [(900, 203, 117), (6000, 64, 48), (4000, 333, 250)])
+def test_hidden_candidates_dropped(ctx, n, W, H, tuning):
+    """Overdraw from tens to thousands of faces a tile, tiles across the image's edges, ties
+    and special depths, cleared buffers and a given depth buffer, both pipelines: frames
+    drawn without statistics equal the oracle's bit for bit."""
+    scene, args = overdraw_scene(n, W, H, n)
+    given = np.random.default_rng(n).uniform(-0.3, 1.0, (H, W)).astype(np.float32)
+    given[::7, ::5] = 0.25
+    mesh = ctx.upload(scene)
+    try:
+        for depth in (None, given):
+            f = None if depth is None else np.full((3, H, W), 7, np.uint8)
+            ref = oracle.draw_frame(scene, args, frame=f, depth=depth)
+            for fused in (True, False):
+                got = _draw_plain(ctx, mesh, scene, args, depth, fused, tuning)
+                _assert_frame(got, ref, f"n {n} {W}x{H} {tuning} depth {depth is not None} fused {fused}")
+    finally:
+        mesh.close()
+
+
+def test_hidden_candidates_dropped_wide_frame_and_batch(ctx):
+    """The same with 64-thread workgroups (a frame of 16,384 tiles) and in a batch, as five
+    launches and as one."""
+    big, bargs = scenes.large_triangle_scene(n=900, size=2048)
+    ref = oracle.draw_frame(big, bargs)
+    mesh = ctx.upload(big)
+    try:
+        _assert_frame(_draw_plain(ctx, mesh, big, bargs, None), ref, "2048x2048")
+    finally:
+        mesh.close()
+    work = [overdraw_scene(5000, 120, 90, 1), scenes.large_triangle_scene(n=500, size=300), overdraw_scene(300, 80, 80, 2)]
+    refs = [oracle.draw_frame(s, a) for s, a in work]
+    meshes = [ctx.upload(s) for s, _ in work]
+    outs = [tuple(ctx.empty(sh, t) for sh, t in (((3, a.image_height, a.image_width), np.uint8),
+                                                 ((a.image_height, a.image_width), np.float32),
+                                                 ((a.image_height, a.image_width), np.int32))) for _, a in work]
+    batch = [(m, s.lights_copy(), a, *o) for m, (s, a), o in zip(meshes, work, outs)]
+    try:
+        for persistent in (False, True):
+            for tuning in ((16, 0), (16, 8192), (8, 0), (32, 0)):
+                ctx.set_batch_persistent(persistent)
+                ctx.set_tuning(*tuning)
+                ctx.draw_batch(batch)
+                for k, (o, ref) in enumerate(zip(outs, refs)):
+                    _assert_frame([b.download() for b in o], ref, f"batch item {k} persistent {persistent} {tuning}")
+    finally:
+        ctx.set_batch_persistent(False)
+        ctx.set_tuning(16, 0)
+        for m in meshes:
+            m.close()
+        for o in outs:
+            for b in o:
+                b.close()
 
 
 @pytest.mark.parametrize("W,H", [(300, 200), (2048, 2048)])
