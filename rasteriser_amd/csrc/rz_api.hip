@@ -91,7 +91,7 @@ struct rz_mesh {
     // from here and the bin pass gathers nothing (uniform = 1)
     int32_t uniform = 0, uniform_n = 0, uniform_t = -1, uniform_m = 0;
     float uniform_nrm[3] = {0.f, 0.f, 0.f};   // model-space normal uniform_n
-    bool overdrawn = false;                   // mesh_overdrawn
+    double layers = 0.0;                      // mesh_layers
     DevMaterial* mats = nullptr;
     uint32_t* texels = nullptr;
     float* luts = nullptr;
@@ -380,6 +380,21 @@ rz_status check_frame(rz_ctx* ctx, const rz_mesh* mesh, const rz_light* lights, 
     return RZ_OK;
 }
 
+// RasterParams::overdrawn: faces covering their extent (mesh_layers) more often than this.
+constexpr double kOverdrawn = 2.0;
+
+// BinParams::parts: up to 16 for a frame whose binning would occupy a quarter of the CUs or
+// less and whose faces, drawn to fill it, meet kWideFace tiles or more each.  (3,000
+// screen-sized triangles: bin pass 199 us in one part, 37 in 16; a 960-face sphere at
+// 512x512, half a tile a face, 9.7 us in one part and 11.1 in 16: the other parts only
+// repeat its transform.)
+constexpr double kWideFace = 4.0;
+uint32_t frame_bin_parts(int32_t nf, double layers, int32_t ntiles) {
+    const uint32_t b = frame_bin_blocks(nf);
+    if (b == 0 || b > 64 || layers * ntiles < kWideFace * nf) return 1;
+    return std::min(512u / b, 16u);
+}
+
 // Builds matrices and light directions (written back to `lights`, as drawing.cpp:238
 // does) and fills every pass's parameters over the working buffers `buf`.
 // Single frames use generation `gen` of the counter lines (and zero the other one).
@@ -448,6 +463,7 @@ void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args
     bp.part_front = part + lay.off_front;
     bp.part_pairs = part + lay.off_pairs;
     bp.nf = mesh->nf; bp.W = lay.W; bp.H = lay.H;
+    bp.parts = frame_bin_parts(mesh->nf, mesh->layers, lay.ntiles);
     bp.tiles_x = lay.tiles_x; bp.ts_log2 = lay.tsl; bp.cap = lay.cap;
     bp.wind_cw = a.wind_clockwise != 0;
     bp.ntiles = lay.ntiles;
@@ -484,7 +500,7 @@ void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args
     rp.ovf_list = bp.ovf_list;
     rp.front_mask = bp.front_mask;
     rp.face_v = mesh->bin_face_v;
-    rp.overdrawn = mesh->overdrawn ? 1 : 0;
+    rp.overdrawn = mesh->layers > kOverdrawn ? 1 : 0;
     rp.max_blocks = lay.raster_grid;
     L.orp = rp;   // batches: k_overflow_batch
     L.orp.part_frag = part + lay.off_ovf;
@@ -556,7 +572,7 @@ void frame_shape(const rz_ctx* ctx, const rz_mesh* mesh, const rz_args& a, int m
              ((a.image_height + ctx->tile_size - 1) / ctx->tile_size);
     narrow = ctx->tile_size == 16 && ntiles >= kNarrowTiles;
     const uint32_t per_cu =
-        raster_blocks_per_cu(ctx->tile_size, ctx->fused, mode, narrow, (flags & RZ_FLAG_CLEARED) == 0, mesh->overdrawn);
+        raster_blocks_per_cu(ctx->tile_size, ctx->fused, mode, narrow, (flags & RZ_FLAG_CLEARED) == 0, mesh->layers > kOverdrawn);
     grid = (uint32_t)ctx->cus * per_cu / 8u * 8u;
     if (grid < 8) grid = 8;
 }
@@ -680,6 +696,7 @@ rz_status counts_ready(rz_ctx* ctx, int32_t ntiles, int gen) {
     if (ctx->count_ptr == ctx->tile_count.ptr && ctx->count_ntiles == ntiles && ctx->count_gen == gen) return RZ_OK;
     BinParams z;
     std::memset(&z, 0, sizeof z);
+    z.parts = 1;
     z.zero_count = count_lines(ntiles);
     z.zero_lines = (uint32_t*)ctx->tile_count.ptr + (size_t)gen * z.zero_count * kCountStride;
     z.zero_blocks = (z.zero_count + kFrameBinBlock - 1) / kFrameBinBlock;
@@ -1446,15 +1463,13 @@ void bin_faces(const rz_mesh_desc* d, std::vector<BinFace>& out) {
     }
 }
 
-// Whether a view of the mesh is likely to cover its pixels several times: the faces' total
-// area against the surface of the box their centroids spread over (model space), or against
-// its screen rectangle (raster space).  Seen from anywhere, front faces show about a quarter
+// How many times the faces cover their extent: their total area over the surface of the box
+// their centroids spread over (model space), or over its screen rectangle (raster space).  Seen from anywhere, front faces show about a quarter
 // of the area and the box a quarter of its surface, so the ratio is about the depth
 // complexity over the box: 0.5 for a sphere, tens for triangle soups.  (A side of the box:
 // the uniform distribution's 2 sqrt(3) standard deviations, which a few far vertices barely
 // move.)
-constexpr double kOverdrawn = 2.0;
-bool mesh_overdrawn(const rz_mesh_desc* d) {
+double mesh_layers(const rz_mesh_desc* d) {
     const int stride = d->raster_space ? 4 : 3, dims = d->raster_space ? 2 : 3;
     double area = 0.0, sum[3] = {0, 0, 0}, sq[3] = {0, 0, 0};
     for (int32_t f = 0; f < d->num_faces; ++f) {
@@ -1476,7 +1491,8 @@ bool mesh_overdrawn(const rz_mesh_desc* d) {
     for (int c = 0; c < dims; ++c) side[c] = std::sqrt(12.0 * std::max(0.0, sq[c] / n - (sum[c] / n) * (sum[c] / n)));
     const double box = d->raster_space ? side[0] * side[1]
                                        : 2.0 * (side[0] * side[1] + side[1] * side[2] + side[2] * side[0]);
-    return area > kOverdrawn * box;   // (false for NaN)
+    const double r = area / box;   // (infinite for faces around one point)
+    return r > 0.0 ? r : 0.0;      // (NaN: 0)
 }
 
 }  // namespace
@@ -1495,7 +1511,7 @@ rz_status rz_mesh_create(rz_ctx* ctx, const rz_mesh_desc* d, rz_mesh** out) {
     m->nf = d->num_faces;
     m->nm = d->num_materials;
     m->raster_space = d->raster_space != 0;
-    m->overdrawn = mesh_overdrawn(d);
+    m->layers = mesh_layers(d);
     auto cleanup = [&](rz_status s) {
         rz_mesh_destroy(ctx, m);
         return s;
@@ -2451,6 +2467,7 @@ rz_status rz_draw_frame_noalloc(rz_ctx* ctx, const rz_mesh* mesh, rz_light* ligh
     // start at zero, by a fill kernel
     BinParams z;
     std::memset(&z, 0, sizeof z);
+    z.parts = 1;
     z.zero_count = count_lines(lay.ntiles);
     z.zero_lines = (uint32_t*)ptrs[kBufTiles];
     z.zero_blocks = (z.zero_count + kFrameBinBlock - 1) / kFrameBinBlock;

@@ -276,11 +276,14 @@ __device__ __forceinline__ bool shrink_rect(const float4& a, const float4& b, co
 template <int BLOCK>
 struct BinLds {
     static constexpr int kAggTiles = 4 * BLOCK;
-    static constexpr int kBytes = 2 * kAggTiles * 4 + BLOCK * kBigTriangleTiles + 24;
+    static constexpr int kBytes = 2 * kAggTiles * 4 + BLOCK * kBigTriangleTiles + 40;
 };
 
-template <int BLOCK>
-__device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned char* lds) {
+// part of parts: this workgroup's share of the faces that are binned by windows of tiles
+// (below); part 0 does everything else.
+template <int BLOCK, bool PARTS = false>
+__device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned char* lds, int part_ = 0, int parts_ = 1) {
+    const int part = PARTS ? part_ : 0, parts = PARTS ? parts_ : 1;
     // faces are taken in the mesh's binning order (centroid Morton order), so the
     // workgroup's faces are screen neighbours; f is the face's own index
     const int i = blk * BLOCK + threadIdx.x;
@@ -293,7 +296,8 @@ __device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned c
         // (none for a mesh whose faces all share them): two dependent round trips, not three
         const int4 q0 = p.face_v[i];
         int4 q1 = make_int4(0, 0, 0, 0), q2 = q1;
-        if (p.gather) {
+        const bool gather = p.gather && part == 0;
+        if (gather) {
             q1 = p.face_attr[2 * i];
             q2 = p.face_attr[2 * i + 1];
         }
@@ -304,7 +308,7 @@ __device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned c
         float4 n0 = make_float4(0.f, 0.f, 0.f, 0.f), n1 = n0, n2 = n0;
         float2 t0 = make_float2(0.f, 0.f), t1 = t0, t2 = t0;
         int32_t mat = 0;
-        if (p.gather) {
+        if (gather) {
             const float4* nsrc = p.nrm ? p.nrm : p.cnormal;
             n0 = nsrc[p.flat ? f : q1.x]; n1 = nsrc[p.flat ? f : q1.y]; n2 = nsrc[p.flat ? f : q1.z];
             if (q2.x >= 0) t0 = p.uvs[q2.x];
@@ -317,7 +321,7 @@ __device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned c
             b = raster_vertex(p.camera, b.x, b.y, b.z, p.Wf, p.Hf);
             c = raster_vertex(p.camera, c.x, c.y, c.z, p.Wf, p.Hf);
         }
-        if (p.gather && p.nrm) {
+        if (gather && p.nrm) {
             n0 = camera_normal(p.normal, n0.x, n0.y, n0.z);
             n1 = p.flat ? n0 : camera_normal(p.normal, n1.x, n1.y, n1.z);
             n2 = p.flat ? n0 : camera_normal(p.normal, n2.x, n2.y, n2.z);
@@ -343,11 +347,13 @@ __device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned c
         // a record only for a face with pixels to raster (a culled face, or one whose box
         // holds no pixel, is never read: the mask below leaves it out)
         if (front && tlx <= brx && tly <= bry) {
-            r->r0 = make_float4(a.x, a.y, a.z, area);
-            r->r1 = make_float4(b.x, b.y, b.z, __uint_as_float(tlx | (tly << 16)));
-            r->r2 = make_float4(c.x, c.y, c.z, __uint_as_float(brx | (bry << 16)));
-            r->r3 = make_float4(a.w, b.w, c.w, 0.0f);
-            if (p.gather) {
+            if (part == 0) {
+                r->r0 = make_float4(a.x, a.y, a.z, area);
+                r->r1 = make_float4(b.x, b.y, b.z, __uint_as_float(tlx | (tly << 16)));
+                r->r2 = make_float4(c.x, c.y, c.z, __uint_as_float(brx | (bry << 16)));
+                r->r3 = make_float4(a.w, b.w, c.w, 0.0f);
+            }
+            if (gather) {
                 r->r4 = make_float4(n0.x, n0.y, n0.z, t0.x);
                 r->r5 = make_float4(n1.x, n1.y, n1.z, t0.y);
                 r->r6 = make_float4(n2.x, n2.y, n2.z, t1.x);
@@ -361,31 +367,34 @@ __device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned c
         // the wave's 64 binning positions (blk * BLOCK is a multiple of 64): the faces
         // with a record
         const unsigned long long fm = __ballot(tx0 <= tx1 && ty0 <= ty1);
-        if ((threadIdx.x & 63) == 0 && i < p.nf) p.front_mask[(uint32_t)i >> 6] = fm;
+        if ((threadIdx.x & 63) == 0 && i < p.nf && part == 0) p.front_mask[(uint32_t)i >> 6] = fm;
     }
     const uint32_t nt = (tx0 <= tx1 && ty0 <= ty1) ? (tx1 - tx0 + 1) * (ty1 - ty0 + 1) : 0u;
     const bool big = nt > (uint32_t)kBigTriangleTiles;
-    const bool small = nt > 0 && !big;
+    bool small = nt > 0 && !big;
 
     // Small faces: aggregate the workgroup's (tile, face) pairs in LDS so that each
     // distinct tile costs one device-scope atomic per workgroup, all issued at once.
     // Faces of one workgroup are neighbours in the mesh, so their tiles usually fall in
     // a small rectangle; when the union of their tile rectangles is larger than
-    // kAggTiles the pairs go to the tile counters one by one.
+    // kAggTiles they are binned by windows with the large faces (below), or, scattered over
+    // a large image, their pairs go to the tile counters one by one.
     constexpr int kAggTiles = BinLds<BLOCK>::kAggTiles;
     uint32_t* s_cnt = reinterpret_cast<uint32_t*>(lds);
     uint32_t* s_base = s_cnt + kAggTiles;
     uint8_t* s_slot = reinterpret_cast<uint8_t*>(s_base + kAggTiles);
-    // union tile rect x0 y0 x1 y1, then the workgroup's front faces and (face, tile) pairs
+    // union tile rect x0 y0 x1 y1 of the small faces, then of the big ones, then the
+    // workgroup's front faces and (face, tile) pairs
     int* s_rect = reinterpret_cast<int*>(s_slot + BLOCK * kBigTriangleTiles);
-    uint32_t* s_stat = reinterpret_cast<uint32_t*>(s_rect + 4);
+    int* s_wide = s_rect + 4;
+    uint32_t* s_stat = reinterpret_cast<uint32_t*>(s_wide + 4);
     const int tid = threadIdx.x;
-    if (tid == 0) {
-        s_rect[0] = s_rect[1] = 0x7FFFFFFF;
-        s_rect[2] = s_rect[3] = -1;
-        s_stat[0] = s_stat[1] = 0u;
-    }
+    if (tid < 10) s_rect[tid] = tid >= 8 ? 0 : (tid & 2) ? -1 : 0x7FFFFFFF;
     __syncthreads();
+    if (big) {   // (few faces, or few workgroups)
+        atomicMin(&s_wide[0], (int)tx0); atomicMin(&s_wide[1], (int)ty0);
+        atomicMax(&s_wide[2], (int)tx1); atomicMax(&s_wide[3], (int)ty1);
+    }
     {
         // union of the small faces' tile rectangles and the statistics' partial sums: per
         // wave, then one LDS atomic each (one exchange for both)
@@ -406,14 +415,27 @@ __device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned c
         }
     }
     __syncthreads();
-    if (tid == 0) {
+    if (tid == 0 && part == 0) {
         p.part_front[blk] = s_stat[0];
         p.part_pairs[blk] = s_stat[1];
     }
-    const int ux0 = s_rect[0], uy0 = s_rect[1];
-    const int uw = s_rect[2] - ux0 + 1, uh = s_rect[3] - uy0 + 1;
-    const bool agg = s_rect[2] >= 0 && uw * uh <= kAggTiles;   // uniform over the workgroup
-    if (agg) {
+    const int4 ur = *reinterpret_cast<const int4*>(s_rect);
+    const int ux0 = ur.x, uy0 = ur.y, uw = ur.z - ux0 + 1, uh = ur.w - uy0 + 1;
+    const bool agg = ur.z >= 0 && uw * uh <= kAggTiles;   // uniform over the workgroup
+    bool wide = false;   // a small face binned by windows
+    int4 wr = *reinterpret_cast<const int4*>(s_wide);
+    if (!agg && ur.z >= 0) {
+        // the small faces too by windows, unless those are many (faces scattered over a
+        // large image)
+        const int4 u = make_int4(min(wr.x, ur.x), min(wr.y, ur.y), max(wr.z, ur.z), max(wr.w, ur.w));
+        if ((u.z - u.x + 1) * (u.w - u.y + 1) <= 8 * parts * kAggTiles) {
+            wide = small;
+            small = false;
+            wr = u;
+        }
+    }
+    small = small && part == 0;
+    if (agg && part == 0) {
         const int area = uw * uh;
         for (int i = tid; i < area; i += BLOCK) s_cnt[i] = 0u;
         __syncthreads();
@@ -448,20 +470,67 @@ __device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned c
         for (uint32_t ty = ty0; ty <= ty1; ++ty)
             for (uint32_t tx = tx0; tx <= tx1; ++tx) bin_push(p, (uint32_t)f, ty * p.tiles_x + tx);
     }
-    // Faces meeting many tiles are binned by the whole wave, one face at a time.
-    unsigned long long bm = __ballot(big);
-    while (bm) {
-        const int src = __ffsll((long long)bm) - 1;
-        bm &= bm - 1;
-        // (src is uniform: lane reads, not LDS permutes)
-        const uint32_t bx0 = __builtin_amdgcn_readlane(tx0, src), bx1 = __builtin_amdgcn_readlane(tx1, src);
-        const uint32_t by0 = __builtin_amdgcn_readlane(ty0, src), by1 = __builtin_amdgcn_readlane(ty1, src);
-        const uint32_t bf = __builtin_amdgcn_readlane((uint32_t)f, src);
-        const uint32_t w = bx1 - bx0 + 1, n = w * (by1 - by0 + 1);
-        for (uint32_t k = lane_id(); k < n; k += 64) {
-            const uint32_t ty = by0 + k / w, tx = bx0 + k % w;
-            bin_push(p, bf, ty * p.tiles_x + tx);
+    // Faces meeting many tiles: by windows of at most kAggTiles tiles of their union
+    // rectangle.  Each wave spreads its lanes over the tiles of one large face in the window,
+    // face after face (a lane goes over a small face's alone), first counting in LDS, then, with one device-scope atomic per tile
+    // of the window, taking its slots from LDS too.  A frame of few faces has `parts`
+    // workgroups for the same faces, each with its own windows (BinParams::parts).  (One
+    // returning device atomic per face and tile instead, a round trip per 64 tiles of every
+    // face: 3,000 screen-sized triangles at 1024x1024, 24 workgroups, 380 us.)
+    if (wr.z < 0) return;   // (uniform)
+    const int bx0 = wr.x, by0 = wr.y, bx1 = wr.z, by1 = wr.w;
+    const int ww = min(bx1 - bx0 + 1, kAggTiles), rows = by1 - by0 + 1;
+    const int wh = min(kAggTiles / ww, (rows + parts - 1) / parts);
+    const int nx = (bx1 - bx0 + ww) / ww, nwin = nx * ((rows + wh - 1) / wh);
+    for (int win = part; win < nwin; win += parts) {
+        const int wx0 = bx0 + win % nx * ww, wy0 = by0 + win / nx * wh;
+        const int wx1 = min(wx0 + ww - 1, bx1), wy1 = min(wy0 + wh - 1, by1);
+        const int cw = wx1 - wx0 + 1, area = cw * (wy1 - wy0 + 1);
+        auto each = [&](auto visit) {   // (face, tile) of this wave's faces in the window
+            if (wide) {
+                for (int y = max((int)ty0, wy0); y <= min((int)ty1, wy1); ++y)
+                    for (int x = max((int)tx0, wx0); x <= min((int)tx1, wx1); ++x)
+                        visit((uint32_t)f, (y - wy0) * cw + (x - wx0), (uint32_t)y * p.tiles_x + (uint32_t)x);
+            }
+            unsigned long long bm = __ballot(big && (int)tx0 <= wx1 && (int)tx1 >= wx0 && (int)ty0 <= wy1 && (int)ty1 >= wy0);
+            while (bm) {
+                const int src = __ffsll((long long)bm) - 1;
+                bm &= bm - 1;
+                // (src is uniform: lane reads, not LDS permutes)
+                const int x0 = max((int)__builtin_amdgcn_readlane(tx0, src), wx0);
+                const int x1 = min((int)__builtin_amdgcn_readlane(tx1, src), wx1);
+                const int y0 = max((int)__builtin_amdgcn_readlane(ty0, src), wy0);
+                const int y1 = min((int)__builtin_amdgcn_readlane(ty1, src), wy1);
+                const uint32_t bf = __builtin_amdgcn_readlane((uint32_t)f, src);
+                const uint32_t w = x1 - x0 + 1, n = w * (y1 - y0 + 1);
+                const float rw = __builtin_amdgcn_rcpf((float)w);
+                for (uint32_t k = lane_id(); k < n; k += 64) {
+                    // k / w exactly: |error| of the product < 1 / (2 w) for k < 1024
+                    const uint32_t dy = (uint32_t)(((float)k + 0.5f) * rw);
+                    const int x = x0 + (int)(k - dy * w), y = y0 + (int)dy;
+                    visit(bf, (y - wy0) * cw + (x - wx0), (uint32_t)y * p.tiles_x + (uint32_t)x);
+                }
+            }
+        };
+        for (int k = tid; k < area; k += BLOCK) s_cnt[k] = 0u;
+        __syncthreads();
+        each([&](uint32_t, int k, uint32_t) { atomicAdd(&s_cnt[k], 1u); });
+        __syncthreads();
+        for (int k = tid; k < area; k += BLOCK) {
+            const uint32_t c = s_cnt[k];
+            if (!c) continue;
+            const uint32_t tile = (uint32_t)(wy0 + k / cw) * p.tiles_x + (uint32_t)(wx0 + k % cw);
+            const uint32_t base = atomicAdd(&p.tile_count[(size_t)tile * kCountStride], c);
+            s_cnt[k] = base;
+            if (base == 0) list_tile(p, tile);
+            if (base <= p.cap && base + c > p.cap) tile_overflowed(p, tile);
         }
+        __syncthreads();
+        each([&](uint32_t face, int k, uint32_t tile) {
+            const uint32_t slot = atomicAdd(&s_cnt[k], 1u);
+            if (slot < p.cap) p.bins[(size_t)tile * p.cap + slot] = face;
+        });
+        __syncthreads();
     }
 }
 
@@ -1482,11 +1551,13 @@ __device__ __forceinline__ void zero_lines_body(const BinParams& p, uint32_t blk
 // (fused pipeline, cleared buffers) the clearing ones, which run on the CUs the
 // latency-bound binning leaves idle.
 // (single frames: kFrameBinBlock-thread workgroups)
+template <bool PARTS>
 __global__ __launch_bounds__(kFrameBinBlock) void k_bin(BinParams p) {
     __shared__ __align__(16) unsigned char s_lds[BinLds<kFrameBinBlock>::kBytes];
-    const uint32_t nb = frame_bin_blocks(p.nf);
+    const uint32_t parts = PARTS ? p.parts : 1u;
+    const uint32_t nb = frame_bin_blocks(p.nf) * parts;
     if (blockIdx.x < nb)
-        bin_body<kFrameBinBlock>(p, blockIdx.x, s_lds);
+        bin_body<kFrameBinBlock, PARTS>(p, blockIdx.x / parts, s_lds, blockIdx.x % parts, parts);
     else if (blockIdx.x < nb + p.zero_blocks)
         zero_lines_body<kFrameBinBlock>(p, blockIdx.x - nb);
     else
@@ -2162,8 +2233,12 @@ hipError_t launch_hold(uint64_t ticks, hipStream_t s) {
 }
 
 hipError_t launch_bin(const BinParams& p, hipStream_t s) {
-    const uint32_t blocks = frame_bin_blocks(p.nf) + p.zero_blocks + (p.clear_np ? p.clear_blocks : 0u);
-    if (blocks) hipLaunchKernelGGL(k_bin, dim3(blocks), dim3(kFrameBinBlock), 0, s, p);
+    const uint32_t blocks = frame_bin_blocks(p.nf) * p.parts + p.zero_blocks + (p.clear_np ? p.clear_blocks : 0u);
+    if (!blocks) return hipSuccess;
+    if (p.parts > 1)
+        hipLaunchKernelGGL(k_bin<true>, dim3(blocks), dim3(kFrameBinBlock), 0, s, p);
+    else
+        hipLaunchKernelGGL(k_bin<false>, dim3(blocks), dim3(kFrameBinBlock), 0, s, p);
     return hipGetLastError();
 }
 

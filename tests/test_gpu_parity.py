@@ -154,6 +154,32 @@ def test_hidden_candidates_dropped_wide_frame_and_batch(ctx):
                 b.close()
 
 
+@pytest.mark.parametrize("tile,cap", [(8, 0), (16, 0), (32, 0), (16, 5)])
+@pytest.mark.parametrize("wide,tiny", [(1, 0), (40, 0), (300, 200), (6, 9000)])
+def test_faces_meeting_many_tiles(ctx, wide, tiny, tile, cap):
+    """Faces far larger than the windows of tiles the bin pass takes them by (one face, several
+    workgroups per block of faces, faces of a handful of tiles scattered between them, and
+    too many faces for more than one workgroup per block), with and without overflowing
+    bins: frames, face ids, depths and counts equal the oracle's."""
+    W, H = 1500, 700
+    rng = np.random.default_rng(wide + tiny)
+    n = wide + tiny
+    c = rng.uniform(0, 1, (n, 1, 2)) * [W, H]
+    rad = np.where(np.arange(n) < wide, rng.uniform(60, 2500, n), rng.uniform(2, 30, n))[:, None, None]
+    xy = c + rad * rng.uniform(-1, 1, (n, 3, 2))
+    verts = np.concatenate([xy, rng.uniform(0, 1, (n, 3, 1)), np.ones((n, 3, 1))], 2).reshape(-1, 4).astype(np.float32)
+    tri = np.arange(3 * n).reshape(n, 3)
+    scene = Scene(verts, np.array([[0.0, 0.0, 1.0]], np.float32), np.zeros((1, 2), np.float32),
+                  make_faces(tri, n=np.zeros_like(tri), t=None), [MaterialSpec((0.9, 0.8, 0.7))],
+                  make_lights([[0.0, 0.0, -1.0]], [200.0 * np.pi], [[1.0, 0.9, 0.8]]), raster_space=True)
+    gpu, ref = check(ctx, scene, make_args(W, H), tuning=(tile, cap), label=f"{wide} wide {tiny} tiny tile {tile} cap {cap}")
+    mesh = ctx.upload(scene)
+    try:
+        _assert_frame(_draw_plain(ctx, mesh, scene, make_args(W, H), None, True, (tile, cap)), ref, "without statistics")
+    finally:
+        mesh.close()
+
+
 @pytest.mark.parametrize("W,H", [(300, 200), (2048, 2048)])
 def test_not_cleared_buffers(ctx, W, H):
     """draw_frame does not clear: the depth test reads the existing depth and pixels it
