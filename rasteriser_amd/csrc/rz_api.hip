@@ -408,8 +408,8 @@ void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args
     L.ext_lights.assign(nl > kMaxLights ? 6 * (size_t)(nl - kMaxLights) : 0, 0.0f);
     for (int32_t l = 0; l < nl; ++l) {
         light_direction(mats.view, lights[l].direction, lights[l].trans_dir);   // drawing.cpp:238
-        float* ic = l < kMaxLights ? L.sp.light_ic[l] : &L.ext_lights[6 * (size_t)(l - kMaxLights)];
-        float* nd = l < kMaxLights ? L.sp.light_nd[l] : ic + 3;
+        float* ic = l < kMaxLights ? L.sp.lights[l].ic : &L.ext_lights[6 * (size_t)(l - kMaxLights)];
+        float* nd = l < kMaxLights ? L.sp.lights[l].nd : ic + 3;
         for (int c = 0; c < 3; ++c) {
             ic[c] = lights[l].intensity * lights[l].colour[c];
             nd[c] = -lights[l].trans_dir[c];
@@ -2467,7 +2467,6 @@ rz_status rz_draw_frame_noalloc(rz_ctx* ctx, const rz_mesh* mesh, rz_light* ligh
     // start at zero, by a fill kernel
     BinParams z;
     std::memset(&z, 0, sizeof z);
-    z.parts = 1;
     z.zero_count = count_lines(lay.ntiles);
     z.zero_lines = (uint32_t*)ptrs[kBufTiles];
     z.zero_blocks = (z.zero_count + kFrameBinBlock - 1) / kFrameBinBlock;

@@ -204,6 +204,14 @@ struct BatchLists {
 };
 
 struct ShadeParams {
+// A light in the kernel arguments: one 32-byte scalar load.
+struct alignas(32) LightParam {
+    float nd[3];   // -trans_dir
+    float pad0;
+    float ic[3];   // intensity * colour
+    float pad1;
+};
+
     const unsigned long long* vis;
     const FaceRecord* rec;
     const DevMaterial* mats;
@@ -235,8 +243,7 @@ struct ShadeParams {
     uint32_t max_blocks;             // persistent strip kernel: workgroups to launch (0 = one per strip)
     int32_t pre_cleared;             // empty pixels already hold 0 / 1.0 / -1 (bin launch cleared them)
     float normal_mat[16];            // inverse-transpose of the model-view (tangents)
-    float light_ic[kMaxLights][3];   // intensity * colour per light
-    float light_nd[kMaxLights][3];   // -trans_dir per light
+    LightParam lights[kMaxLights];
     // lights kMaxLights .. nl-1 (nl > kMaxLights only): (intensity * colour, -trans_dir),
     // six floats per light, in device memory
     const float* lights_ext;
