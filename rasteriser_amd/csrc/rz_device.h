@@ -118,8 +118,9 @@ struct BinParams {
     uint32_t* part_front;       // per workgroup: front faces
     uint32_t* part_pairs;       // per workgroup: (front face, tile) pairs
     int32_t nf;
-    // Workgroups per block of faces (single frames): the parts share the windows of tiles that
-    // faces meeting many tiles are binned by; every part transforms the block's faces.
+    // Single frames: 0, or the workgroups per block of faces of the launch that bins faces
+    // meeting many tiles by windows of tiles; the parts share the windows, every part
+    // transforms the block's faces.
     uint32_t parts;
     uint32_t W, H;
     int32_t tiles_x;
@@ -201,6 +202,14 @@ struct BatchLists {
     const uint32_t* ovf_list;   // those tiles, (mesh << kListMeshShift) | tile
     uint32_t* part_frag;        // per raster workgroup: fragments passing the inside test
     uint32_t* part_cov;         // per raster workgroup, then per overflow-shade workgroup: covered pixels
+};
+
+// A light in the kernel arguments: one 32-byte scalar load.
+struct alignas(32) LightParam {
+    float nd[3];   // -trans_dir
+    float pad0;
+    float ic[3];   // intensity * colour
+    float pad1;
 };
 
 struct ShadeParams {
