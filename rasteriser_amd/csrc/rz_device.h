@@ -118,9 +118,8 @@ struct BinParams {
     uint32_t* part_front;       // per workgroup: front faces
     uint32_t* part_pairs;       // per workgroup: (front face, tile) pairs
     int32_t nf;
-    // Single frames: 0, or the workgroups per block of faces of the launch that bins faces
-    // meeting many tiles by windows of tiles; the parts share the windows, every part
-    // transforms the block's faces.
+    // Workgroups per block of faces (single frames): the parts share the windows of tiles that
+    // faces meeting many tiles are binned by; every part transforms the block's faces.
     uint32_t parts;
     uint32_t W, H;
     int32_t tiles_x;
@@ -213,14 +212,6 @@ struct alignas(32) LightParam {
 };
 
 struct ShadeParams {
-// A light in the kernel arguments: one 32-byte scalar load.
-struct alignas(32) LightParam {
-    float nd[3];   // -trans_dir
-    float pad0;
-    float ic[3];   // intensity * colour
-    float pad1;
-};
-
     const unsigned long long* vis;
     const FaceRecord* rec;
     const DevMaterial* mats;
