@@ -383,16 +383,18 @@ rz_status check_frame(rz_ctx* ctx, const rz_mesh* mesh, const rz_light* lights, 
 // RasterParams::overdrawn: faces covering their extent (mesh_layers) more often than this.
 constexpr double kOverdrawn = 2.0;
 
-// BinParams::parts: up to 16 for a frame whose binning would occupy a quarter of the CUs or
-// less and whose faces, drawn to fill it, meet kWideFace tiles or more each.  (3,000
-// screen-sized triangles: bin pass 199 us in one part, 37 in 16; a 960-face sphere at
-// 512x512, half a tile a face, 9.7 us in one part and 11.1 in 16: the other parts only
-// repeat its transform.)
-constexpr double kWideFace = 4.0;
+// BinParams::parts.  Faces are binned by windows where one, drawn to fill the frame with the
+// others, meets kWideFace tiles or more: elsewhere the few that do are not worth that
+// launch's larger code (1080p icosphere frame, a fifth of a tile a face, 0.2-0.4 us; the
+// 4M-triangle frame 0.7%).  Where binning would occupy a quarter of the CUs or less, up to 16
+// workgroups share a block's windows.  (3,000 screen-sized triangles at 1024x1024: bin pass
+// 382 us by atomics, 199 by windows in one part, 37 in 16; a 960-face sphere at 512x512,
+// half a tile a face, 9.7 by atomics and 11.1 in 16 parts.)
+constexpr double kWideFace = 2.0;
 uint32_t frame_bin_parts(int32_t nf, double layers, int32_t ntiles) {
     const uint32_t b = frame_bin_blocks(nf);
-    if (b == 0 || b > 64 || layers * ntiles < kWideFace * nf) return 1;
-    return std::min(512u / b, 16u);
+    if (b == 0 || layers * ntiles < kWideFace * nf) return 0;
+    return b > 64 ? 1u : std::min(512u / b, 16u);
 }
 
 // Builds matrices and light directions (written back to `lights`, as drawing.cpp:238
@@ -696,7 +698,6 @@ rz_status counts_ready(rz_ctx* ctx, int32_t ntiles, int gen) {
     if (ctx->count_ptr == ctx->tile_count.ptr && ctx->count_ntiles == ntiles && ctx->count_gen == gen) return RZ_OK;
     BinParams z;
     std::memset(&z, 0, sizeof z);
-    z.parts = 1;
     z.zero_count = count_lines(ntiles);
     z.zero_lines = (uint32_t*)ctx->tile_count.ptr + (size_t)gen * z.zero_count * kCountStride;
     z.zero_blocks = (z.zero_count + kFrameBinBlock - 1) / kFrameBinBlock;
@@ -2467,7 +2468,6 @@ rz_status rz_draw_frame_noalloc(rz_ctx* ctx, const rz_mesh* mesh, rz_light* ligh
     // start at zero, by a fill kernel
     BinParams z;
     std::memset(&z, 0, sizeof z);
-    z.parts = 1;
     z.zero_count = count_lines(lay.ntiles);
     z.zero_lines = (uint32_t*)ptrs[kBufTiles];
     z.zero_blocks = (z.zero_count + kFrameBinBlock - 1) / kFrameBinBlock;

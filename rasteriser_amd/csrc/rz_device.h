@@ -118,8 +118,9 @@ struct BinParams {
     uint32_t* part_front;       // per workgroup: front faces
     uint32_t* part_pairs;       // per workgroup: (front face, tile) pairs
     int32_t nf;
-    // Workgroups per block of faces (single frames): the parts share the windows of tiles that
-    // faces meeting many tiles are binned by; every part transforms the block's faces.
+    // Single frames: 0, or the workgroups per block of faces of the launch that bins faces
+    // meeting many tiles by windows of tiles; the parts share the windows, every part
+    // transforms the block's faces.
     uint32_t parts;
     uint32_t W, H;
     int32_t tiles_x;
