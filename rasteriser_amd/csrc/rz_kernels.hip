@@ -1217,7 +1217,7 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
 
     static_assert(BLOCK % 64 == 0, "candidates are dealt in whole waves");
     int par = 0;
-    for (uint32_t base = 0; base < n; base += BLOCK, par ^= 1) {
+    for (uint32_t base = 0; n > 0; par ^= 1) {
         // The chunk's faces (entry base + tid of the bin) into the LDS face table by rank:
         // their candidate rectangles, the prefix sums, the chunk's total of pairs.
         uint32_t cnt = 0, rect = 0;
@@ -1404,8 +1404,10 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
             }
         }
         __syncthreads();       // ranks and wave totals are rewritten by the next chunk
+        base += BLOCK;
+        if (base >= n) break;   // (uniform)
         // the next chunk's records, read here so that none are live through the candidates
-        const uint32_t i = base + BLOCK + (uint32_t)tid;
+        const uint32_t i = base + (uint32_t)tid;
         face = 0u;
         a = b = c = make_float4(0.f, 0.f, 0.f, 0.f);
         if (i < n) {
@@ -1413,7 +1415,7 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
             const FaceRecord* r = p.rec + face;
             a = r->r0; b = r->r1; c = r->r2;
         }
-        if (may_drop && base + BLOCK < n) read_zfar();
+        if (may_drop) read_zfar();
     }
     ahead.entry();
     if (overflowed) return;
