@@ -2172,6 +2172,23 @@ hipError_t launch_copy(const void* src, void* dst, size_t n16, hipStream_t s) {
     return hipGetLastError();
 }
 
+// Device memory to pinned host memory (both 16-byte aligned).  The link bounds it, 55 GB/s, so
+// one workgroup per CU is plenty; being a kernel of the stream it starts when the frame's last kernel
+// ends, where the copy engine's hand-over costs tens of microseconds a chunk.
+__global__ __launch_bounds__(256) void k_download(const uint4* __restrict__ src, uint4* __restrict__ dst,
+                                                  size_t bytes) {
+    const size_t n16 = bytes / 16, stride = (size_t)gridDim.x * 256;
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+    for (size_t i = t; i < n16; i += stride) dst[i] = src[i];
+    if (t < bytes % 16)
+        reinterpret_cast<unsigned char*>(dst)[16 * n16 + t] = reinterpret_cast<const unsigned char*>(src)[16 * n16 + t];
+}
+
+hipError_t launch_download(const unsigned char* src, unsigned char* pinned, size_t bytes, hipStream_t s) {
+    hipLaunchKernelGGL(k_download, dim3(256), dim3(256), 0, s, (const uint4*)src, (uint4*)pinned, bytes);
+    return hipGetLastError();
+}
+
 // ---------------------------------------------------------------------------------
 // Text into a planar frame: the spin loop's frame-rate line (renderer.cpp:114,
 // CImg::draw_text(5, 5, text, white, black)).  Glyphs are this library's own 5x7 bitmaps

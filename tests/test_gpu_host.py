@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import oracle
+import rasteriser_amd as rz
 from rasteriser_amd import scenes
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -123,3 +124,24 @@ def test_renderer_cli_frame_matches_oracle(tmp_path, case):
         got[box] = 0
         want[box] = 0
     assert np.array_equal(got, want), "frame.png differs from the oracle's frame"
+
+
+@pytest.mark.parametrize("nbytes", [1, (4 << 20) - 1, 4 << 20, (16 << 20) + 5, (50 << 20) + 13])
+def test_downloads_through_pinned_chunks(nbytes):
+    """Downloads below the staged size, of a few chunks, of more chunks than the staging
+    holds, ragged at the end, and from an address the staging kernel does not take: the
+    bytes that were uploaded, and nothing written past them."""
+    rng = np.random.default_rng(nbytes)
+    data = rng.integers(0, 256, nbytes, dtype=np.uint8)
+    with rz.Context(0) as c:
+        a = c.empty((nbytes,), np.uint8)
+        a.upload(data)
+        for start in (0, 3):
+            n = nbytes - start
+            if n < 1:
+                continue
+            out = np.full(n + 64, 0xA5, np.uint8)
+            assert c.lib.rz_copy_to_host(c.handle, out.ctypes.data, C.c_void_p(a.ptr + start), n) == 0
+            assert np.array_equal(out[:n], data[start:]), f"{nbytes} bytes from {start}"
+            assert (out[n:] == 0xA5).all()
+        a.close()
