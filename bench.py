@@ -42,7 +42,8 @@ tex texels, P_listed pixels of the tiles the raster pass visits):
   raster   fused: 48 T_front + 4 P16 + 7 C + 108 T_vis + 4 tex + 40 L
            separate: 48 T_front + 4 P16 + 8 P_listed (visibility words written)
   shade    separate: 8 W H + 7 W H + 108 T_vis + 4 tex + 40 L
-  vertex   (batches) 28 V + 24 Vn
+  vertex   (batches: the launch that clears the counters) 8 W H / 256, a pair of words
+           per 16x16 tile
 """
 from __future__ import annotations
 
@@ -306,11 +307,11 @@ def batched(ctx, rz, scenes, np, frames):
         T = sum(sc.num_faces for sc, _ in work)
         L = sum(sc.lights.shape[0] for sc, _ in work)
         pixels = sum(a.image_width * a.image_height for _, a in work)
-        nbytes = {"vertex": 28 * V + 24 * Vn,
-                  "bin": 12 * T + 16 * V + 4 * p16 + 7 * pixels,
+        nbytes = {"vertex": 8 * (pixels // 256),
+                  "bin": 12 * T + 12 * V + 12 * Vn + 4 * p16 + 7 * pixels,
                   "raster": 48 * st["front_triangles"] + 4 * p16 + 7 * st["covered_pixels"] + 108 * vis + 40 * L,
                   "overflow": 0, "shade": 0}
-        names = {"vertex": "k_vertex_batch", "bin": "k_bin_batch", "raster": "k_raster_shade_batch",
+        names = {"vertex": "k_counts_batch", "bin": "k_bin_batch", "raster": "k_raster_shade_batch",
                  "overflow": "k_overflow_batch", "shade": "k_shade_tiles_batch"}
         table = pass_table(med, nbytes, names)
         return {"workload": "256 meshes, log-uniform 500-200k faces, viewports 256^2-1024^2",

@@ -147,8 +147,8 @@ typedef struct rz_frame_stats {
     uint64_t fragments;           /* (pixel, front face) pairs passing the inside test (drawing.cpp:111) */
     uint64_t covered_pixels;      /* pixels holding a winning fragment                       */
     float ms_vertex;              /* GPU time per pass, HIP events on the context stream;    */
-    float ms_bin;                 /* zero unless rz_set_profiling(ctx, 1) (ms_vertex: batches */
-                                  /* only; a single frame's bin pass does the transform)    */
+    float ms_bin;                 /* zero unless rz_set_profiling(ctx, 1) (ms_vertex: a    */
+                                  /* batch's counter clears; 0 for single frames)            */
     float ms_raster;
     float ms_overflow;
     float ms_shade;
@@ -313,15 +313,15 @@ typedef struct rz_batch_item {
 
 /* No reference counterpart (the reference draws one mesh per call).  Draws every
  * item as rz_draw_frame would (bit for bit).  By default a batch frame is five
- * launches, each running one pass of every item (vertex transform; binning and buffer
- * clears; raster-and-shade of the tiles of all items; the overflow loop of tiles whose
+ * launches, each running one pass of every item (counter clears; vertex transform,
+ * binning and buffer clears; raster-and-shade of the tiles of all items; the overflow loop of tiles whose
  * bins overflowed; their shade); with rz_set_batch_persistent it is one launch of a
  * resident grid that runs those passes as phases between grid barriers.  At most 1024
  * items.  Requires RZ_FLAG_DEVICE_BUFFERS; RZ_FLAG_CLEARED and RZ_FLAG_ASYNC apply to
  * all items.  stats (may be NULL) sums over the items; with rz_set_profiling its ms_*
  * are the passes' times (five launches: HIP events between them) or the phases' spans
- * inside the one launch (first start to last end; they overlap; ms_vertex 0, the bin
- * phase transforms the vertices), and ms_frame the whole frame. */
+ * inside the one launch (first start to last end; they overlap; ms_vertex 0, nothing
+ * is cleared there), and ms_frame the whole frame. */
 rz_status rz_draw_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t num_items, uint32_t flags,
                         rz_frame_stats* stats);
 /* 1: a batch frame is one persistent launch (every workgroup resident; a wait that

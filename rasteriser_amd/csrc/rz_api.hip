@@ -24,7 +24,7 @@ hipError_t launch_raster(const RasterParams& p, int tile_size, hipStream_t s);
 hipError_t launch_raster_shade(const RasterParams& p, const ShadeParams& sp, int tile_size, hipStream_t s);
 hipError_t launch_shade_tiles(const RasterParams& p, const ShadeParams& sp, int tile_size, hipStream_t s);
 hipError_t launch_shade(const ShadeParams& p, hipStream_t s);
-hipError_t launch_vertex_batch(const VertexParams* items, const uint2* map, uint32_t blocks, hipStream_t s);
+hipError_t launch_counts_batch(const CountParams* items, const uint2* map, uint32_t blocks, hipStream_t s);
 hipError_t launch_bin_batch(const BinParams* items, const uint2* map, uint32_t blocks, hipStream_t s);
 hipError_t launch_overflow_batch(const RasterParams* items, const uint2* map, uint32_t blocks, hipStream_t s);
 uint32_t raster_batch_blocks_per_cu(int tile_size, int mode);
@@ -82,13 +82,9 @@ struct rz_mesh {
     int device = 0;
     int32_t nv = 0, nn = 0, nt = 0, nf = 0, nm = 0;
     bool raster_space = false;
-    float *px = nullptr, *py = nullptr, *pz = nullptr;
-    float4* rin = nullptr;
-    // (x, y, z, 0) copies for the single-frame bin pass, which transforms each face's
-    // corners itself: positions, vertex normals, face normals
+    float4* rin = nullptr;            // raster-space positions as given
+    // (x, y, z, 0): positions, vertex normals, face normals (flat)
     float4 *pos4 = nullptr, *nrm4 = nullptr, *fnrm4 = nullptr;
-    float *nx = nullptr, *ny = nullptr, *nz = nullptr;      // vertex normals
-    float *fnx = nullptr, *fny = nullptr, *fnz = nullptr;   // face normals (flat)
     float *ftx = nullptr, *fty = nullptr, *ftz = nullptr;   // face tangents (normal maps)
     float2* uvs = nullptr;
     // the faces' indices in binning order: sorted by the Morton code of their centroid
@@ -131,7 +127,7 @@ struct rz_ctx {
     size_t auto_bin_bytes = 0;        // automatic bin capacity: the most bytes of bins (rz_create)
     hipEvent_t ev[6] = {};
     std::string err;
-    DevBuf raster, cnormal, rec, tile_count, bins, vis, lists, frame, depth, ids, counters, partials;
+    DevBuf rec, tile_count, bins, vis, lists, frame, depth, ids, counters, partials;
     DevBuf batch_arena, batch_tables;
     // learned shader: FP32 parameters, Adam moments, packed BF16 network, training scratch
     DevBuf mlp_w, mlp_m, mlp_v, mlp_packed, mlp_gpart, mlp_lpart, mlp_loss, mlp_count;
@@ -396,20 +392,18 @@ struct FrameLayout {
     int ts = 16, tsl = 4, tiles_x = 0, tiles_y = 0, ntiles = 0;
     bool fused = false;     // raster pass shades non-overflowed tiles
     bool batch = false;     // one mesh of a batch (tile lists and raster statistics shared)
-    // two generations of counter lines and no vertex pass (single frames, and the meshes
-    // of a batch's persistent launch): the bin pass transforms each face's corners and
-    // zeroes the other generation
+    // two generations of counter lines (single frames, and the meshes of a batch's
+    // persistent launch): the bin pass zeroes the other generation
     bool twogen = true;
     uint32_t raster_grid = 0, tiles_grid = 0;   // workgroups of the list-driven launches
     uint32_t W = 0, H = 0, cap = 0;
     size_t np = 0;
-    int32_t nfn = 0;
     // per-workgroup statistics sections (uint32 each)
     size_t off_front = 0, off_pairs = 0, off_frag = 0, off_ovf = 0, off_cov = 0, n_part = 0;
-    size_t bytes[9] = {};   // raster, cnormal, rec, tile_count, bins, vis, lists, counters, partials
+    size_t bytes[7] = {};   // rec, tile_count, bins, vis, lists, counters, partials
 };
 
-enum { kBufRaster, kBufCnormal, kBufRec, kBufTiles, kBufBins, kBufVis, kBufLists, kBufCounters, kBufPart, kNumBufs };
+enum { kBufRec, kBufTiles, kBufBins, kBufVis, kBufLists, kBufCounters, kBufPart, kNumBufs };
 
 // Single frame: raster_grid / tiles_grid workgroups of the list-driven raster and
 // overflow-shade launches.  Batch meshes (batch = true) are always fused; the batch owns
@@ -432,7 +426,6 @@ FrameLayout layout_frame(const rz_mesh* mesh, const rz_args& a, int ts, int cap,
     L.tiles_y = (int)((L.H + ts - 1) / ts);
     L.ntiles = L.tiles_x * L.tiles_y;
     L.np = (size_t)L.W * L.H;
-    L.nfn = a.flat ? mesh->nf : mesh->nn;
     L.off_front = 0;
     const size_t nbin = batch ? bin_blocks(mesh->nf, bblock) : frame_bin_blocks(mesh->nf);   // bin workgroups
     L.off_pairs = L.off_front + nbin;
@@ -442,12 +435,9 @@ FrameLayout layout_frame(const rz_mesh* mesh, const rz_args& a, int ts, int cap,
     L.n_part = L.off_cov + (batch ? 0
                                   : L.fused ? (size_t)raster_grid + tiles_grid
                                             : (size_t)shade_blocks_x(L.W) * shade_blocks_y(L.H));
-    // batches: the vertex pass's outputs (raster space: read as given), one generation
-    // of tile counts + the 8 list counters, and the global counters apart.  Single frames
-    // transform in the bin pass and keep two generations of counter lines (count_lines):
-    // each frame's bin pass zeroes the other one for the next frame.
-    L.bytes[kBufRaster] = batch && !mesh->raster_space ? (size_t)mesh->nv * 16 : 0;
-    L.bytes[kBufCnormal] = batch ? (size_t)L.nfn * 16 : 0;
+    // batches: one generation of tile counts + the 8 list counters, and the global counters
+    // apart.  Single frames keep two generations of counter lines (count_lines): each
+    // frame's bin pass zeroes the other one for the next frame.
     // the face records, then the bin pass's front mask (a bit per face)
     L.bytes[kBufRec] = (size_t)mesh->nf * sizeof(FaceRecord) + ((size_t)mesh->nf + 63) / 64 * 8;
     L.bytes[kBufTiles] = batch ? ((size_t)L.ntiles + 8) * 4 * kCountStride
@@ -481,7 +471,7 @@ FrameLayout layout_batch_sync(const rz_mesh* mesh, const rz_args& a, int ts, int
 
 // One frame's kernel parameters, built on the host before anything is enqueued.
 struct FrameLaunch {
-    VertexParams vp;
+    CountParams cp;   // batches
     BinParams bp;
     RasterParams rp;
     RasterParams orp;   // the overflow pass: rp with its own statistics section
@@ -554,40 +544,19 @@ void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args
     L.counters = counters;
     L.gen = gen;
 
-    VertexParams& vp = L.vp;
-    std::memset(&vp, 0, sizeof vp);
-    std::memcpy(vp.camera, mats.camera, 64);
-    std::memcpy(vp.normal, mats.normal, 64);
-    vp.px = mesh->px; vp.py = mesh->py; vp.pz = mesh->pz;
-    vp.nx = a.flat ? mesh->fnx : mesh->nx;
-    vp.ny = a.flat ? mesh->fny : mesh->ny;
-    vp.nz = a.flat ? mesh->fnz : mesh->nz;
-    vp.raster = (float4*)buf[kBufRaster];
-    vp.cnormal = (float4*)buf[kBufCnormal];
-    vp.tile_count = tile_count;
-    vp.counters = counters;
-    // (batches only: single frames transform in the bin pass)
-    vp.nv = mesh->nv; vp.nn = lay.nfn; vp.ntiles = lay.ntiles + 8;   // clears the list counters too
-    // raster-space vertices need no vertex stage: the bin pass reads them where they are
-    if (mesh->raster_space) {
-        vp.nv = 0;
-        vp.raster = mesh->rin;
-    }
-    vp.Wf = (float)lay.W; vp.Hf = (float)lay.H;
+    L.cp = CountParams{tile_count, counters, lay.ntiles + 8};   // the list counters too
 
     BinParams& bp = L.bp;
     std::memset(&bp, 0, sizeof bp);
     bp.face_v = mesh->bin_face_v;
     bp.face_attr = mesh->bin_face_attr;
-    bp.raster = vp.raster;
-    bp.cnormal = vp.cnormal;
     bp.uvs = mesh->uvs;
     bp.flat = a.flat != 0;
     const bool uniform = mesh->uniform && !a.flat;
     bp.gather = uniform ? 0 : 1;
     bp.rec = (FaceRecord*)buf[kBufRec];
     bp.front_mask = (unsigned long long*)(bp.rec + mesh->nf);
-    bp.tile_count = vp.tile_count;
+    bp.tile_count = tile_count;
     bp.bins = (uint32_t*)buf[kBufBins];
     bp.counters = counters;
     bp.part_front = part + lay.off_front;
@@ -601,15 +570,14 @@ void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args
     bp.ovf_list = bp.lists ? bp.lists + (size_t)8 * lay.ntiles : nullptr;
     bp.list_count = bp.tile_count + (size_t)lay.ntiles * kCountStride;
     bp.ovf_vis = (unsigned long long*)buf[kBufVis];
+    // the bin pass transforms each face's corners
+    bp.pos = mesh->raster_space ? nullptr : mesh->pos4;
+    bp.raster = mesh->raster_space ? mesh->rin : nullptr;
+    bp.nrm = a.flat ? mesh->fnrm4 : mesh->nrm4;
+    std::memcpy(bp.camera, mats.camera, 64);
+    std::memcpy(bp.normal, mats.normal, 64);
+    bp.Wf = (float)lay.W; bp.Hf = (float)lay.H;
     if (lay.twogen) {
-        // no vertex pass: the bin pass transforms each face's corners
-        bp.pos = mesh->raster_space ? nullptr : mesh->pos4;
-        bp.raster = mesh->raster_space ? mesh->rin : nullptr;
-        bp.nrm = a.flat ? mesh->fnrm4 : mesh->nrm4;
-        bp.cnormal = nullptr;
-        std::memcpy(bp.camera, mats.camera, 64);
-        std::memcpy(bp.normal, mats.normal, 64);
-        bp.Wf = (float)lay.W; bp.Hf = (float)lay.H;
         bp.zero_lines = (uint32_t*)buf[kBufTiles] + (1 - gen) * gen_words;
         bp.zero_count = count_lines(lay.ntiles);
         bp.zero_blocks = (bp.zero_count + kFrameBinBlock - 1) / kFrameBinBlock;
@@ -736,7 +704,7 @@ rz_status prepare_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
     const bool can_overflow = (uint32_t)cap < (uint32_t)mesh->nf;
     const FrameLayout lay = layout_frame(mesh, *args, ctx->tile_size, cap, ctx->fused, grid,
                                          can_overflow ? ctx->persistent_blocks : 0u, false);
-    DevBuf* bufs[kNumBufs] = {&ctx->raster, &ctx->cnormal, &ctx->rec,   &ctx->tile_count, &ctx->bins,
+    DevBuf* bufs[kNumBufs] = {&ctx->rec,   &ctx->tile_count, &ctx->bins,
                               &ctx->vis,    &ctx->lists,   &ctx->counters, &ctx->partials};
     void* ptrs[kNumBufs];
     for (int i = 0; i < kNumBufs; ++i) {
@@ -903,7 +871,7 @@ struct BatchLaunch {
     std::vector<uint64_t> faces;
     int ts = 16;
     int mode = kShadePlain;
-    const VertexParams* d_vp = nullptr;
+    const CountParams* d_cp = nullptr;
     const BinParams* d_bp = nullptr;
     const RasterParams* d_rp = nullptr;
     const RasterParams* d_orp = nullptr;
@@ -992,7 +960,7 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
         L.sp.mlp = (const uint16_t*)ctx->mlp_packed.ptr;
         bind_outputs(L, cleared, it.frame, it.depth, it.ids);
         L.rp.count_frags = stats ? 1 : 0;
-        // the shared lists; their 8 counters are the first mesh's (cleared by its vertex pass)
+        // the shared lists; their 8 counters are the first mesh's (cleared by the first launch)
         const FrameLaunch& L0 = B.frames[0];
         L.bp.lists = lists;
         L.bp.list_count = L0.bp.list_count;
@@ -1004,7 +972,7 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
         L.rp.list_count = L.orp.list_count = L0.bp.list_count;
         L.rp.ovf_list = L.orp.ovf_list = L.bp.ovf_list;
         B.faces[i] = (uint64_t)it.mesh->nf;
-        const uint32_t nb[3] = {vertex_blocks(L.vp.nv, L.vp.nn, L.vp.ntiles, bblock),
+        const uint32_t nb[3] = {((uint32_t)L.cp.lines + 255u) / 256u,
                                 bin_blocks(L.bp.nf, bblock) + L.bp.clear_blocks, overflow_blocks(L.rp.nf, bblock)};
         for (int p = 0; p < 3; ++p)
             for (uint32_t b = 0; b < nb[p]; ++b)
@@ -1024,7 +992,7 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
     B.bl.part_cov = batch_part + B.raster_grid;
     // tables: the four parameter arrays and the three block maps
     size_t off[7], total = 0;
-    const size_t sz[4] = {sizeof(VertexParams), sizeof(BinParams), sizeof(RasterParams), sizeof(ShadeParams)};
+    const size_t sz[4] = {sizeof(CountParams), sizeof(BinParams), sizeof(RasterParams), sizeof(ShadeParams)};
     for (int p = 0; p < 4; ++p) {
         off[p] = total;
         total = align256(total + sz[p] * (size_t)n);
@@ -1055,7 +1023,7 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
                         B.frames[i].ext_lights.size() * sizeof(float));
     (void)off_ext;
     for (int32_t i = 0; i < n; ++i) {
-        std::memcpy(host.data() + off[0] + i * sz[0], &B.frames[i].vp, sz[0]);
+        std::memcpy(host.data() + off[0] + i * sz[0], &B.frames[i].cp, sz[0]);
         std::memcpy(host.data() + off[1] + i * sz[1], &B.frames[i].bp, sz[1]);
         std::memcpy(host.data() + off[2] + i * sz[2], &B.frames[i].rp, sz[2]);
         std::memcpy(host.data() + off[3] + i * sz[3], &B.frames[i].sp, sz[3]);
@@ -1067,7 +1035,7 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
     RZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
     RZ_HIP(ctx, hipMemcpy(tables.ptr, host.data(), total, hipMemcpyHostToDevice));
     char* t = (char*)tables.ptr;
-    B.d_vp = (const VertexParams*)(t + off[0]);
+    B.d_cp = (const CountParams*)(t + off[0]);
     B.d_bp = (const BinParams*)(t + off[1]);
     B.d_rp = (const RasterParams*)(t + off[2]);
     B.d_sp = (const ShadeParams*)(t + off[3]);
@@ -1258,7 +1226,7 @@ rz_status enqueue_batch(rz_ctx* ctx, const BatchLaunch& B, hipStream_t s, bool p
     }
     if (prof) RZ_HIP(ctx, launch_hold(kHoldTicks, s));
     if (prof) RZ_HIP(ctx, hipEventRecord(ctx->ev[0], s));
-    RZ_HIP(ctx, launch_vertex_batch(B.d_vp, B.d_map[0], B.blocks[0], s));
+    RZ_HIP(ctx, launch_counts_batch(B.d_cp, B.d_map[0], B.blocks[0], s));
     if (prof) RZ_HIP(ctx, hipEventRecord(ctx->ev[1], s));
     RZ_HIP(ctx, launch_bin_batch(B.d_bp, B.d_map[1], B.blocks[1], s));
     if (prof) RZ_HIP(ctx, hipEventRecord(ctx->ev[2], s));
@@ -1431,7 +1399,7 @@ void rz_destroy(rz_ctx* ctx) {
     if (!ctx) return;
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-    DevBuf* bufs[] = {&ctx->raster, &ctx->cnormal, &ctx->rec,   &ctx->tile_count, &ctx->bins,
+    DevBuf* bufs[] = {&ctx->rec,   &ctx->tile_count, &ctx->bins,
                       &ctx->vis,    &ctx->lists,   &ctx->frame,   &ctx->depth, &ctx->ids,        &ctx->counters,
                       &ctx->partials, &ctx->batch_arena, &ctx->batch_tables, &ctx->mlp_w, &ctx->mlp_m,
                       &ctx->mlp_v, &ctx->mlp_packed, &ctx->mlp_gpart, &ctx->mlp_lpart, &ctx->mlp_loss,
@@ -1649,8 +1617,7 @@ rz_status rz_mesh_create(rz_ctx* ctx, const rz_mesh_desc* d, rz_mesh** out) {
     };
     const size_t V = (size_t)m->nv, N = (size_t)m->nn, F = (size_t)m->nf;
     // The faces in binning order; vertices, normals and uvs are renumbered by first use
-    // in that order, so that the bin pass reads them (and a batch's vertex pass writes
-    // them) in address order.  Only storage moves: every value and face index is the caller's.
+    // in that order, so that the bin pass reads them in address order.  Only storage moves: every value and face index is the caller's.
     std::vector<BinFace> faces;
     bin_faces(d, faces);
     std::vector<int32_t> vorder, norder, torder;   // new index -> caller's index
@@ -1673,43 +1640,30 @@ rz_status rz_mesh_create(rz_ctx* ctx, const rz_mesh_desc* d, rz_mesh** out) {
         for (size_t i = 0; i < N; ++i) if (nmap[i] < 0) norder.push_back((int32_t)i);
         for (size_t i = 0; i < tmap.size(); ++i) if (tmap[i] < 0) torder.push_back((int32_t)i);
     }
-    // positions: (x, y, z, 0) per vertex for the single-frame bin pass, SoA for a batch's
-    // coalesced vertex pass
     if (m->raster_space) {
         std::vector<float> rv(4 * V);
         for (size_t i = 0; i < V; ++i)
             for (int c = 0; c < 4; ++c) rv[4 * i + c] = d->vertices[4 * (size_t)vorder[i] + c];
         if ((st = upload(ctx, m, &m->rin, rv.data(), V * 16)) != RZ_OK) return cleanup(st);
     } else {
-        std::vector<float> sx(V), sy(V), sz(V);
-        for (size_t i = 0; i < V; ++i) {
-            const size_t o = (size_t)vorder[i];
-            sx[i] = d->vertices[3 * o];
-            sy[i] = d->vertices[3 * o + 1];
-            sz[i] = d->vertices[3 * o + 2];
-        }
-        if ((st = upload(ctx, m, &m->px, sx.data(), V * 4)) != RZ_OK) return cleanup(st);
-        if ((st = upload(ctx, m, &m->py, sy.data(), V * 4)) != RZ_OK) return cleanup(st);
-        if ((st = upload(ctx, m, &m->pz, sz.data(), V * 4)) != RZ_OK) return cleanup(st);
         std::vector<float4> p4(V);
-        for (size_t i = 0; i < V; ++i) p4[i] = make_float4(sx[i], sy[i], sz[i], 0.f);
+        for (size_t i = 0; i < V; ++i) {
+            const float* v = d->vertices + 3 * (size_t)vorder[i];
+            p4[i] = make_float4(v[0], v[1], v[2], 0.f);
+        }
         if ((st = upload(ctx, m, &m->pos4, p4.data(), V * 16)) != RZ_OK) return cleanup(st);
         // face normals for flat shading, model space
-        std::vector<float> fx(F), fy(F), fz(F);
+        std::vector<float4> f4(F);
         for (size_t f = 0; f < F; ++f) {
             const rz_triangle& t = d->faces[f];
             float nrm[3];
             face_normal(d->vertices + 3 * (size_t)t.vertices[0], d->vertices + 3 * (size_t)t.vertices[1],
                         d->vertices + 3 * (size_t)t.vertices[2], nrm);
-            fx[f] = nrm[0]; fy[f] = nrm[1]; fz[f] = nrm[2];
+            f4[f] = make_float4(nrm[0], nrm[1], nrm[2], 0.f);
         }
-        if ((st = upload(ctx, m, &m->fnx, fx.data(), F * 4)) != RZ_OK) return cleanup(st);
-        if ((st = upload(ctx, m, &m->fny, fy.data(), F * 4)) != RZ_OK) return cleanup(st);
-        if ((st = upload(ctx, m, &m->fnz, fz.data(), F * 4)) != RZ_OK) return cleanup(st);
-        std::vector<float4> f4(F);
-        for (size_t f = 0; f < F; ++f) f4[f] = make_float4(fx[f], fy[f], fz[f], 0.f);
         if ((st = upload(ctx, m, &m->fnrm4, f4.data(), F * 16)) != RZ_OK) return cleanup(st);
         // face tangents for normal maps, model space
+        std::vector<float> fx(F), fy(F), fz(F);
         for (size_t f = 0; f < F; ++f) {
             const rz_triangle& t = d->faces[f];
             float tc[3][2] = {{0.f, 0.f}, {0.f, 0.f}, {0.f, 0.f}};
@@ -1728,18 +1682,11 @@ rz_status rz_mesh_create(rz_ctx* ctx, const rz_mesh_desc* d, rz_mesh** out) {
         if ((st = upload(ctx, m, &m->ftz, fz.data(), F * 4)) != RZ_OK) return cleanup(st);
     }
     {
-        std::vector<float> sx(N), sy(N), sz(N);
-        for (size_t i = 0; i < N; ++i) {
-            const size_t o = (size_t)norder[i];
-            sx[i] = d->normals[3 * o];
-            sy[i] = d->normals[3 * o + 1];
-            sz[i] = d->normals[3 * o + 2];
-        }
-        if ((st = upload(ctx, m, &m->nx, sx.data(), N * 4)) != RZ_OK) return cleanup(st);
-        if ((st = upload(ctx, m, &m->ny, sy.data(), N * 4)) != RZ_OK) return cleanup(st);
-        if ((st = upload(ctx, m, &m->nz, sz.data(), N * 4)) != RZ_OK) return cleanup(st);
         std::vector<float4> n4(N);
-        for (size_t i = 0; i < N; ++i) n4[i] = make_float4(sx[i], sy[i], sz[i], 0.f);
+        for (size_t i = 0; i < N; ++i) {
+            const float* v = d->normals + 3 * (size_t)norder[i];
+            n4[i] = make_float4(v[0], v[1], v[2], 0.f);
+        }
         if ((st = upload(ctx, m, &m->nrm4, n4.data(), N * 16)) != RZ_OK) return cleanup(st);
     }
     {
@@ -2372,7 +2319,7 @@ rz_status rz_autotune(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32
         std::vector<uint32_t> counts;
         for (const FrameLaunch& L : B.frames) {
             counts.resize(L.lay.ntiles);
-            RZ_HIP(ctx, hipMemcpy2DAsync(counts.data(), 4, L.vp.tile_count, 4 * kCountStride, 4, counts.size(),
+            RZ_HIP(ctx, hipMemcpy2DAsync(counts.data(), 4, L.cp.tile_count, 4 * kCountStride, 4, counts.size(),
                                          hipMemcpyDeviceToHost, ctx->stream));
             RZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
             for (uint32_t c : counts) need = c > need ? c : need;

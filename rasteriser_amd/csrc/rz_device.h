@@ -76,17 +76,12 @@ struct DevMaterial {
     uint32_t pad[2];
 };
 
-struct VertexParams {
-    float camera[16];
-    float normal[16];
-    const float* px; const float* py; const float* pz;   // model positions (SoA)
-    const float* nx; const float* ny; const float* nz;   // normals to transform (SoA)
-    float4* raster;                                      // out: (x_px, y_px, ndc_z, 1/w)
-    float4* cnormal;                                     // out: camera-space normal (xyz)
-    uint32_t* tile_count;
+// A batch mesh's counters, cleared before its bin pass (single frames keep two generations
+// and the bin pass clears the other one).
+struct CountParams {
+    uint32_t* tile_count;       // one counter per line (kCountStride), then the 8 list counters
     unsigned long long* counters;
-    int32_t nv, nn, ntiles;
-    float Wf, Hf;
+    int32_t lines;
 };
 
 // A face's indices in the bin pass's order, in two arrays: (v0, v1, v2, face), and
@@ -98,11 +93,10 @@ struct BinFace {
 struct BinParams {
     const int4* face_v;         // (v0, v1, v2, face) in binning order
     const int4* face_attr;      // (n0, n1, n2, material), (t0, t1, t2, 0) in binning order
+    // each face transforms its own corners.  pos (x, y, z, -): model positions (null: `raster`
+    // holds raster-space positions as given); nrm (x, y, z, -): model normals (flat: one per
+    // face)
     const float4* raster;
-    const float4* cnormal;      // camera-space normals (flat: one per face)
-    // Single frames have no vertex pass: each face transforms its own corners.  pos
-    // (x, y, z, -): model positions (null: `raster` holds raster-space positions as
-    // given); nrm (x, y, z, -): model normals (flat: one per face; null: `cnormal`).
     const float4* pos;
     const float4* nrm;
     float camera[16];
@@ -251,14 +245,8 @@ struct ShadeParams {
 };
 
 // Launch shapes (shared by the launchers, the batch block maps and the host's
-// statistics reduction).  `block`: workgroup size of a batch's vertex, bin and overflow
-// work (256, or the persistent batch launch's batch_block).
-__host__ __device__ inline uint32_t vertex_blocks(int32_t nv, int32_t nn, int32_t ntiles, int block = 256) {
-    int32_t n = nv > nn ? nv : nn;
-    if (ntiles > n) n = ntiles;
-    if (kNumCounters > n) n = kNumCounters;
-    return (uint32_t)((n + block - 1) / block);
-}
+// statistics reduction).  `block`: workgroup size of a batch's bin and overflow work (256,
+// or the persistent batch launch's batch_block).
 __host__ __device__ inline uint32_t bin_blocks(int32_t nf, int block = 256) {
     return (uint32_t)((nf + block - 1) / block);
 }

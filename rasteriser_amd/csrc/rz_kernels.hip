@@ -9,8 +9,8 @@
 //               meets (fixed capacity per tile)
 //               and each tile's first face puts the tile on a per-XCD list; more
 //               workgroups zero the next frame's generation of counter lines.
-//               (Batches run the transform as a vertex pass of their own,
-//               k_vertex_batch, which also clears the meshes' counters.)
+//               (Batches clear their meshes' counters in a launch of its own,
+//               k_counts_batch.)
 //   k_raster    resident grid over the tile lists, one tile per workgroup at a time:
 //               expands (face, box pixel) candidates with wavefront prefix scans,
 //               runs the inside and depth tests of drawing.cpp:96-121 and keeps per
@@ -123,20 +123,6 @@ __device__ __forceinline__ float4 camera_normal(const float* m, float x, float y
     n.z = (m[2] * x + m[6] * y) + (m[10] * z + m[14] * w);
     n.w = 0.0f;
     return n;
-}
-
-// Batches: the vertex pass of every mesh (single frames transform in the bin pass).
-template <int BLOCK = 256>
-__device__ __forceinline__ void vertex_body(const VertexParams& p, int blk) {
-    const int i = blk * BLOCK + threadIdx.x;
-    if (i < p.nv)   // (raster-space meshes have nv = 0: the bin pass reads their vertices)
-        p.raster[i] = raster_vertex(p.camera, p.px[i], p.py[i], p.pz[i], p.Wf, p.Hf);
-    if (i < p.nn) p.cnormal[i] = camera_normal(p.normal, p.nx[i], p.ny[i], p.nz[i]);
-    if (i < p.ntiles) p.tile_count[(size_t)i * kCountStride] = 0u;
-    // (the last 8 entries are the tile lists' counters; their second word is a batch's
-    // work cursor)
-    if (i + 8 >= p.ntiles && i < p.ntiles) p.tile_count[(size_t)i * kCountStride + 1] = 0u;
-    if (i < kNumCounters) p.counters[i] = 0ull;
 }
 
 // ---------------------------------------------------------------------------------
@@ -310,7 +296,7 @@ __device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned c
         float2 t0 = make_float2(0.f, 0.f), t1 = t0, t2 = t0;
         int32_t mat = 0;
         if (gather) {
-            const float4* nsrc = p.nrm ? p.nrm : p.cnormal;
+            const float4* nsrc = p.nrm;
             n0 = nsrc[p.flat ? f : q1.x]; n1 = nsrc[p.flat ? f : q1.y]; n2 = nsrc[p.flat ? f : q1.z];
             if (q2.x >= 0) t0 = p.uvs[q2.x];
             if (q2.y >= 0) t1 = p.uvs[q2.y];
@@ -322,7 +308,7 @@ __device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned c
             b = raster_vertex(p.camera, b.x, b.y, b.z, p.Wf, p.Hf);
             c = raster_vertex(p.camera, c.x, c.y, c.z, p.Wf, p.Hf);
         }
-        if (gather && p.nrm) {
+        if (gather) {
             n0 = camera_normal(p.normal, n0.x, n0.y, n0.z);
             n1 = p.flat ? n0 : camera_normal(p.normal, n1.x, n1.y, n1.z);
             n2 = p.flat ? n0 : camera_normal(p.normal, n2.x, n2.y, n2.z);
@@ -1852,10 +1838,17 @@ __device__ __forceinline__ void take_tiles(const BatchLists& bl, uint32_t* s_tak
     }
 }
 
-__global__ __launch_bounds__(256) void k_vertex_batch(const VertexParams* __restrict__ items,
+// A batch's first launch: every mesh's counters.  (Transforming the meshes' vertices here, for
+// the bin pass to read back, took 60 us of the 128-mesh batch's frame and made its bin pass
+// no faster than transforming each face's corners there: 244 -> 231 us.)
+__global__ __launch_bounds__(256) void k_counts_batch(const CountParams* __restrict__ items,
                                                       const uint2* __restrict__ map) {
     const uint2 m = map[blockIdx.x];
-    vertex_body(items[m.x], (int)m.y);
+    const CountParams& p = items[m.x];
+    const int i = (int)m.y * 256 + threadIdx.x;
+    // (words 0 and 1 of each line: a count, and a list counter's work cursor)
+    if (i < p.lines) *reinterpret_cast<uint2*>(p.tile_count + (size_t)i * kCountStride) = make_uint2(0u, 0u);
+    if (i < kNumCounters) p.counters[i] = 0ull;
 }
 // Batch bin launch: each mesh's binning workgroups, then its clearing ones.
 __global__ __launch_bounds__(256) void k_bin_batch(const BinParams* __restrict__ items, const uint2* __restrict__ map) {
@@ -2470,8 +2463,8 @@ hipError_t launch_shade(const ShadeParams& p, hipStream_t s) {
 
 // Batch launchers: `items` and `map` are device arrays, `blocks` the summed block
 // count of the pass over all meshes.
-hipError_t launch_vertex_batch(const VertexParams* items, const uint2* map, uint32_t blocks, hipStream_t s) {
-    if (blocks) hipLaunchKernelGGL(k_vertex_batch, dim3(blocks), dim3(256), 0, s, items, map);
+hipError_t launch_counts_batch(const CountParams* items, const uint2* map, uint32_t blocks, hipStream_t s) {
+    if (blocks) hipLaunchKernelGGL(k_counts_batch, dim3(blocks), dim3(256), 0, s, items, map);
     return hipGetLastError();
 }
 hipError_t launch_bin_batch(const BinParams* items, const uint2* map, uint32_t blocks, hipStream_t s) {
