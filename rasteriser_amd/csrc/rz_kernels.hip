@@ -1053,10 +1053,13 @@ __device__ __forceinline__ uint32_t bucket_floor(uint32_t bucket, uint32_t near,
 // Overdraw: faces of a later chunk behind the tile's farthest pixel so far are dropped as
 // they are staged, and a chunk of kSortPairs or more is taken roughly front to back, so
 // that a pair whose face lies behind both its pixels is dropped before the edge functions
-// and a wave's remaining pairs once their faces lie behind the farthest pixel.  A face's depth bound is depth_floor's; 64 buckets between the chunk's nearest
-// and farthest bounds order the faces.  Dropped candidates could not have changed a key, so
-// the result is the same; only the count of inside-test fragments needs every one
-// (count_frags: a frame whose caller asked for statistics).
+// and a wave's remaining pairs once their faces lie behind the farthest pixel.  A face's
+// depth bound is depth_floor's; 64 buckets between the chunk's nearest and farthest bounds
+// order the faces.  Dropped candidates could not have changed a key, so the result is the
+// same; only the count of inside-test fragments needs every one (count_frags: a frame whose
+// caller asked for statistics).  What bounds an overdrawn tile is the vector instructions of
+// its candidates: 3,000 screen-sized triangles at 1024x1024 191 -> 77 us for the pass, the
+// raster launch of a 12-mesh batch 186 -> 62 us, of a 128-mesh batch 964 -> 676 us.
 //
 // FUSED: the workgroup then shades its own pixels from the LDS visibility words (the
 // deferred shade, without the round trip of the visibility buffer through HBM).  Tiles
@@ -1078,8 +1081,9 @@ __device__ __forceinline__ TileHead tile_head(const RasterParams& p, int tile, i
     return h;
 }
 
-// A tile of more faces than this may drop hidden candidates; a chunk of at least this many candidate pairs (eight candidates per pixel of the tile)
-// is taken front to back (raster_body).
+// A tile of more than kDropFaces faces (one-wave workgroups: more than a chunk) may drop
+// hidden candidates; a chunk of at least kSortPairs candidate pairs (eight candidates per
+// pixel of the tile) is taken front to back (raster_body).
 constexpr uint32_t kDropFaces = 32;
 template <int NPX>
 constexpr uint32_t kSortPairs = 4 * NPX;

@@ -145,3 +145,22 @@ def test_downloads_through_pinned_chunks(nbytes):
             assert np.array_equal(out[:n], data[start:]), f"{nbytes} bytes from {start}"
             assert (out[n:] == 0xA5).all()
         a.close()
+
+
+def test_download_into_pinned_memory():
+    """A download into memory that is pinned already goes there directly: the same bytes."""
+    nbytes = (5 << 20) + 7
+    data = np.random.default_rng(5).integers(0, 256, nbytes, dtype=np.uint8)
+    with rz.Context(0) as c:
+        hip = C.CDLL("libamdhip64.so.7")   # (the runtime librz is linked to)
+        p = C.c_void_p()
+        assert hip.hipHostMalloc(C.byref(p), C.c_size_t(nbytes + 64), C.c_uint(0)) == 0
+        out = np.ctypeslib.as_array(C.cast(p, C.POINTER(C.c_uint8)), (nbytes + 64,))
+        out[:] = 0xA5
+        a = c.empty((nbytes,), np.uint8)
+        a.upload(data)
+        assert c.lib.rz_copy_to_host(c.handle, p, C.c_void_p(a.ptr), nbytes) == 0
+        assert np.array_equal(out[:nbytes], data) and (out[nbytes:] == 0xA5).all()
+        a.close()
+        del out
+        assert hip.hipHostFree(p) == 0
