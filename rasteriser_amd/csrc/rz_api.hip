@@ -27,14 +27,14 @@ hipError_t launch_shade(const ShadeParams& p, hipStream_t s);
 hipError_t launch_counts_batch(const CountParams* items, const uint2* map, uint32_t blocks, hipStream_t s);
 hipError_t launch_bin_batch(const BinParams* items, const uint2* map, uint32_t blocks, hipStream_t s);
 hipError_t launch_overflow_batch(const RasterParams* items, const uint2* map, uint32_t blocks, hipStream_t s);
-uint32_t raster_batch_blocks_per_cu(int tile_size, int mode);
-uint32_t batch_frame_blocks_per_cu(int tile_size, int mode);
+uint32_t raster_batch_blocks_per_cu(int tile_size, int mode, bool drop);
+uint32_t batch_frame_blocks_per_cu(int tile_size, int mode, bool drop);
 hipError_t launch_batch_frame(const BinParams* b, const RasterParams* r, const RasterParams* o,
                               const ShadeParams* sh, const BatchLists& bl0, const BatchLists& bl1,
-                              const BatchSync& q, int tile_size, int mode, hipStream_t s);
+                              const BatchSync& q, int tile_size, int mode, bool drop, hipStream_t s);
 hipError_t launch_batch_tiles(const RasterParams* items, const ShadeParams* sitems, const BatchLists& bl,
                               uint32_t raster_grid, uint32_t tiles_grid, int tile_size, int mode, hipStream_t s,
-                              bool raster);
+                              bool raster, bool drop);
 hipError_t launch_hold(uint64_t ticks, hipStream_t s);
 hipError_t launch_check_quotients(uint32_t blocks, uint32_t per_thread, uint32_t seed, unsigned long long* counts,
                                   hipStream_t s);
@@ -901,6 +901,7 @@ struct BatchLaunch {
     std::vector<uint64_t> faces;
     int ts = 16;
     int mode = kShadePlain;
+    bool drop = true;               // hidden candidates dropped: no statistics asked for
     const CountParams* d_cp = nullptr;
     const BinParams* d_bp = nullptr;
     const RasterParams* d_rp = nullptr;
@@ -940,8 +941,9 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
     B.ts = ctx->tile_size;
     B.mode = (flags & RZ_FLAG_MLP_SHADE) ? kShadeMlp : kShadePlain;
     B.persistent = false;
+    B.drop = !stats;
     const int bblock = 256;
-    uint32_t grid = (uint32_t)ctx->cus * raster_batch_blocks_per_cu(B.ts, B.mode) / 8u * 8u;
+    uint32_t grid = (uint32_t)ctx->cus * raster_batch_blocks_per_cu(B.ts, B.mode, B.drop) / 8u * 8u;
     B.raster_grid = grid < 8 ? 8 : grid;
     B.tiles_grid = (uint32_t)ctx->persistent_blocks;
     std::vector<FrameLayout> lays(n);
@@ -989,7 +991,6 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
         fill_frame(it.mesh, it.lights, it.num_lights, it.args, flags, lays[i], ptrs, L);
         L.sp.mlp = (const uint16_t*)ctx->mlp_packed.ptr;
         bind_outputs(L, cleared, it.frame, it.depth, it.ids);
-        L.rp.count_frags = stats ? 1 : 0;
         // the shared lists; their 8 counters are the first mesh's (cleared by the first launch)
         const FrameLaunch& L0 = B.frames[0];
         L.bp.lists = lists;
@@ -1091,9 +1092,10 @@ rz_status prepare_batch_sync(rz_ctx* ctx, const rz_batch_item* items, int32_t n,
     B.ts = ctx->tile_size;
     B.mode = (flags & RZ_FLAG_MLP_SHADE) ? kShadeMlp : kShadePlain;
     B.persistent = true;
+    B.drop = !stats;
     const int bblock = batch_block(B.ts);
     // every workgroup of the launch resident at once: the launch's occupancy on every CU
-    uint32_t grid = (uint32_t)ctx->cus * batch_frame_blocks_per_cu(B.ts, B.mode) / 8u * 8u;
+    uint32_t grid = (uint32_t)ctx->cus * batch_frame_blocks_per_cu(B.ts, B.mode, B.drop) / 8u * 8u;
     B.raster_grid = B.tiles_grid = grid < 8 ? 8 : grid;
     const int cap = ctx->bin_cap > 0 ? ctx->bin_cap : kDefaultBinCap;
     std::vector<FrameLayout> lays(n);
@@ -1143,7 +1145,6 @@ rz_status prepare_batch_sync(rz_ctx* ctx, const rz_batch_item* items, int32_t n,
             L.sp.mlp = (const uint16_t*)ctx->mlp_packed.ptr;
             L.sp.mode = B.mode;
             bind_outputs(L, cleared, it.frame, it.depth, it.ids);
-            L.rp.count_frags = stats ? 1 : 0;
             // the shared lists; their 8 counters, and the batch's overflow count, are the
             // first mesh's (its bin work zeroes the other generation's for the next frame)
             const FrameLaunch& L0 = g ? B.frames1[0] : B.frames[0];
@@ -1250,7 +1251,7 @@ rz_status enqueue_batch(rz_ctx* ctx, const BatchLaunch& B, hipStream_t s, bool p
     if (B.persistent) {
         if (prof) RZ_HIP(ctx, launch_hold(kHoldTicks, s));
         if (prof) RZ_HIP(ctx, hipEventRecord(ctx->ev[0], s));
-        RZ_HIP(ctx, launch_batch_frame(B.d_bp, B.d_rp, B.d_orp, B.d_sp, B.bl, B.bl1, B.q, B.ts, B.mode, s));
+        RZ_HIP(ctx, launch_batch_frame(B.d_bp, B.d_rp, B.d_orp, B.d_sp, B.bl, B.bl1, B.q, B.ts, B.mode, B.drop, s));
         if (prof) RZ_HIP(ctx, hipEventRecord(ctx->ev[5], s));
         return RZ_OK;
     }
@@ -1260,11 +1261,11 @@ rz_status enqueue_batch(rz_ctx* ctx, const BatchLaunch& B, hipStream_t s, bool p
     if (prof) RZ_HIP(ctx, hipEventRecord(ctx->ev[1], s));
     RZ_HIP(ctx, launch_bin_batch(B.d_bp, B.d_map[1], B.blocks[1], s));
     if (prof) RZ_HIP(ctx, hipEventRecord(ctx->ev[2], s));
-    RZ_HIP(ctx, launch_batch_tiles(B.d_rp, B.d_sp, B.bl, B.raster_grid, B.tiles_grid, B.ts, B.mode, s, true));
+    RZ_HIP(ctx, launch_batch_tiles(B.d_rp, B.d_sp, B.bl, B.raster_grid, B.tiles_grid, B.ts, B.mode, s, true, B.drop));
     if (prof) RZ_HIP(ctx, hipEventRecord(ctx->ev[3], s));
     RZ_HIP(ctx, launch_overflow_batch(B.d_orp, B.d_map[2], B.blocks[2], s));
     if (prof) RZ_HIP(ctx, hipEventRecord(ctx->ev[4], s));
-    RZ_HIP(ctx, launch_batch_tiles(B.d_rp, B.d_sp, B.bl, B.raster_grid, B.tiles_grid, B.ts, B.mode, s, false));
+    RZ_HIP(ctx, launch_batch_tiles(B.d_rp, B.d_sp, B.bl, B.raster_grid, B.tiles_grid, B.ts, B.mode, s, false, B.drop));
     if (prof) RZ_HIP(ctx, hipEventRecord(ctx->ev[5], s));
     return RZ_OK;
 }
@@ -1950,7 +1951,7 @@ rz_status rz_draw_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
         }
     }
     bind_outputs(L, cleared, frame_d, depth_d, ids_d);
-    L.rp.count_frags = stats ? 1 : 0;
+    if (stats) L.rp.overdrawn = 0;   // (every fragment is counted)
     if ((st = run_frame(ctx, L, ctx->profiling)) != RZ_OK) return st;
     if (!on_device) {
         const Download d[3] = {{frame_buffer, frame_d, np * 3}, {depth_buffer, depth_d, np * 4}, {id_buffer, ids_d, np * 4}};

@@ -1056,8 +1056,8 @@ __device__ __forceinline__ uint32_t bucket_floor(uint32_t bucket, uint32_t near,
 // and a wave's remaining pairs once their faces lie behind the farthest pixel.  A face's
 // depth bound is depth_floor's; 64 buckets between the chunk's nearest and farthest bounds
 // order the faces.  Dropped candidates could not have changed a key, so the result is the
-// same; only the count of inside-test fragments needs every one (count_frags: a frame whose
-// caller asked for statistics).  What bounds an overdrawn tile is the vector instructions of
+// same; only the count of inside-test fragments needs every one, so frames whose caller asks
+// for statistics take the plain variant.  What bounds an overdrawn tile is the vector instructions of
 // its candidates: 3,000 screen-sized triangles at 1024x1024 191 -> 77 us for the pass, the
 // raster launch of a 12-mesh batch 186 -> 62 us, of a 128-mesh batch 964 -> 676 us.
 //
@@ -1163,7 +1163,7 @@ __device__ __forceinline__ void raster_body(const RasterParams& p, const ShadePa
     // fills them: such a tile has no chunk and no stores here (uniform over the workgroup)
     const bool overflowed = count > p.cap;
     const uint32_t n = overflowed ? 0u : count;
-    const bool may_drop = DROP && n > (NW > 1 ? kDropFaces : (uint32_t)BLOCK) && !p.count_frags;   // (uniform)
+    const bool may_drop = DROP && n > (NW > 1 ? kDropFaces : (uint32_t)BLOCK) ;   // (uniform)
     // the first chunk's face records, read before anything waits
     uint32_t face = f_first;
     float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a, c = a;
@@ -1868,7 +1868,9 @@ __global__ __launch_bounds__(256) void k_bin_batch(const BinParams* __restrict__
 // A batch's raster pass: one resident grid over the tile lists the meshes share, entry
 // (mesh << kListMeshShift) | tile, raster and shade of the tile with its mesh's
 // parameters.
-template <int TS, int BLOCK, int MODE>
+// DROP: hidden candidates are dropped (raster_body), in every batch whose caller asks for no
+// statistics.
+template <int TS, int BLOCK, int MODE, bool DROP>
 __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 6) void k_raster_shade_batch(
     const RasterParams* __restrict__ items, const ShadeParams* __restrict__ sitems, BatchLists bl) {
     __shared__ __align__(16) uint16_t s_net[MODE == kShadeMlp ? kPackedBytes / 2 : 8];
@@ -1878,7 +1880,7 @@ __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 6) void k_raster_sha
     take_tiles(bl, s_take, [&](uint32_t e, TakeAhead ahead) {
         const uint32_t m = e >> kListMeshShift;
         const int tile = (int)(e & kListTileMask);
-        raster_body<TS, BLOCK, true, MODE, kShrinkPixels, false, kSlabAlways>(
+        raster_body<TS, BLOCK, true, MODE, kShrinkPixels, false, kSlabAlways, false, DROP>(
             items[m], &sitems[m], nullptr, nullptr, s_net, tile, tile_head(items[m], tile, threadIdx.x), frags,
             cov, nullptr, ahead);
     });
@@ -1959,21 +1961,23 @@ __device__ __forceinline__ void phase_clock(const BatchSync& q, int phase, bool 
     }
 }
 
-template <int BLOCK, int MODE>
+template <int BLOCK, int MODE, bool DROP>
 struct BatchFrameLds {
-    static constexpr int kBytes =
-        BinLds<BLOCK>::kBytes > RasterLds<BLOCK, MODE>::kBytes ? BinLds<BLOCK>::kBytes : RasterLds<BLOCK, MODE>::kBytes;
+    static constexpr int kBytes = BinLds<BLOCK>::kBytes > RasterLds<BLOCK, MODE, DROP>::kBytes
+                                      ? BinLds<BLOCK>::kBytes
+                                      : RasterLds<BLOCK, MODE, DROP>::kBytes;
 };
 
 // bitems / ritems / oitems: nmesh parameter records of generation 0, then of generation 1
 // (their counter lines differ); sitems: one per mesh.
-template <int TS, int BLOCK, int MODE>
+// DROP: as k_raster_shade_batch's.
+template <int TS, int BLOCK, int MODE, bool DROP>
 __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 4) void k_batch_frame(
     const BinParams* __restrict__ bitems, const RasterParams* __restrict__ ritems,
     const RasterParams* __restrict__ oitems, const ShadeParams* __restrict__ sitems, BatchLists bl0,
     BatchLists bl1, BatchSync q) {
     // one LDS region for the bin phase's tile aggregation and the raster phase's face data
-    __shared__ __align__(16) unsigned char s_lds[BatchFrameLds<BLOCK, MODE>::kBytes];
+    __shared__ __align__(16) unsigned char s_lds[BatchFrameLds<BLOCK, MODE, DROP>::kBytes];
     __shared__ __align__(16) uint16_t s_net[MODE == kShadeMlp ? kPackedBytes / 2 : 8];
     __shared__ unsigned long long s_frame;
     __shared__ uint32_t s_take[3];
@@ -2033,7 +2037,7 @@ __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 4) void k_batch_fram
     take_tiles(bl, s_take, [&](uint32_t e, TakeAhead ahead) {
         const uint32_t m = e >> kListMeshShift;
         const int tile = (int)(e & kListTileMask);
-        raster_body<TS, BLOCK, true, MODE, kShrinkPixels, true, kSlabAlways>(
+        raster_body<TS, BLOCK, true, MODE, kShrinkPixels, true, kSlabAlways, false, DROP>(
             ritems[gen * nm + m], &sitems[m], nullptr, nullptr, s_net, tile,
             tile_head(ritems[gen * nm + m], tile, threadIdx.x), frags, cov, s_lds, ahead);
     });
@@ -2114,13 +2118,16 @@ uint32_t resident_blocks_per_cu(const void* f, int block, size_t lds_budget = (s
 }
 
 // Resident workgroups per CU of the persistent batch launch.
-uint32_t batch_frame_blocks_per_cu(int tile_size, int mode) {
+uint32_t batch_frame_blocks_per_cu(int tile_size, int mode, bool drop) {
     const void* f = nullptr;
     int block = 256;
 #define RZ_PICK(TS, B)                                                                               \
     block = B;                                                                                       \
-    f = mode == kShadeMlp ? reinterpret_cast<const void*>(&k_batch_frame<TS, B, kShadeMlp>)           \
-                          : reinterpret_cast<const void*>(&k_batch_frame<TS, B, kShadePlain>);
+    f = mode == kShadeMlp                                                                            \
+            ? (drop ? reinterpret_cast<const void*>(&k_batch_frame<TS, B, kShadeMlp, true>)           \
+                    : reinterpret_cast<const void*>(&k_batch_frame<TS, B, kShadeMlp, false>))         \
+            : (drop ? reinterpret_cast<const void*>(&k_batch_frame<TS, B, kShadePlain, true>)         \
+                    : reinterpret_cast<const void*>(&k_batch_frame<TS, B, kShadePlain, false>));
     switch (tile_size) {
         case 8: RZ_PICK(8, 64) break;
         case 16: RZ_PICK(16, 256) break;
@@ -2132,15 +2139,18 @@ uint32_t batch_frame_blocks_per_cu(int tile_size, int mode) {
 
 hipError_t launch_batch_frame(const BinParams* b, const RasterParams* r, const RasterParams* o,
                               const ShadeParams* sh, const BatchLists& bl0, const BatchLists& bl1,
-                              const BatchSync& q, int tile_size, int mode, hipStream_t s) {
-#define RZ_LAUNCH(TS, B, M) \
-    hipLaunchKernelGGL((k_batch_frame<TS, B, M>), dim3(q.G), dim3(B), 0, s, b, r, o, sh, bl0, bl1, q)
+                              const BatchSync& q, int tile_size, int mode, bool drop, hipStream_t s) {
+#define RZ_LAUNCH(TS, B, M)                                                                             \
+    if (drop)                                                                                           \
+        hipLaunchKernelGGL((k_batch_frame<TS, B, M, true>), dim3(q.G), dim3(B), 0, s, b, r, o, sh, bl0, bl1, q); \
+    else                                                                                                \
+        hipLaunchKernelGGL((k_batch_frame<TS, B, M, false>), dim3(q.G), dim3(B), 0, s, b, r, o, sh, bl0, bl1, q)
     const bool net = mode == kShadeMlp;
     if (mode != kShadePlain && mode != kShadeMlp) return hipErrorInvalidValue;
     switch (tile_size) {
-        case 8: if (net) RZ_LAUNCH(8, 64, kShadeMlp); else RZ_LAUNCH(8, 64, kShadePlain); break;
-        case 16: if (net) RZ_LAUNCH(16, 256, kShadeMlp); else RZ_LAUNCH(16, 256, kShadePlain); break;
-        case 32: if (net) RZ_LAUNCH(32, 256, kShadeMlp); else RZ_LAUNCH(32, 256, kShadePlain); break;
+        case 8: if (net) { RZ_LAUNCH(8, 64, kShadeMlp); } else { RZ_LAUNCH(8, 64, kShadePlain); } break;
+        case 16: if (net) { RZ_LAUNCH(16, 256, kShadeMlp); } else { RZ_LAUNCH(16, 256, kShadePlain); } break;
+        case 32: if (net) { RZ_LAUNCH(32, 256, kShadeMlp); } else { RZ_LAUNCH(32, 256, kShadePlain); } break;
         default: return hipErrorInvalidValue;
     }
 #undef RZ_LAUNCH
@@ -2481,13 +2491,16 @@ hipError_t launch_overflow_batch(const RasterParams* items, const uint2* map, ui
 }
 
 // Resident workgroups per CU of the batch raster kernel.
-uint32_t raster_batch_blocks_per_cu(int tile_size, int mode) {
+uint32_t raster_batch_blocks_per_cu(int tile_size, int mode, bool drop) {
     const void* f = nullptr;
     int block = 256;
 #define RZ_PICK(TS, B)                                                                              \
     block = B;                                                                                      \
-    f = mode == kShadeMlp ? reinterpret_cast<const void*>(&k_raster_shade_batch<TS, B, kShadeMlp>)   \
-                          : reinterpret_cast<const void*>(&k_raster_shade_batch<TS, B, kShadePlain>);
+    f = mode == kShadeMlp                                                                               \
+            ? (drop ? reinterpret_cast<const void*>(&k_raster_shade_batch<TS, B, kShadeMlp, true>)       \
+                    : reinterpret_cast<const void*>(&k_raster_shade_batch<TS, B, kShadeMlp, false>))     \
+            : (drop ? reinterpret_cast<const void*>(&k_raster_shade_batch<TS, B, kShadePlain, true>)     \
+                    : reinterpret_cast<const void*>(&k_raster_shade_batch<TS, B, kShadePlain, false>));
     switch (tile_size) {
         case 8: RZ_PICK(8, 64) break;
         case 16: RZ_PICK(16, 256) break;
@@ -2502,11 +2515,15 @@ uint32_t raster_batch_blocks_per_cu(int tile_size, int mode) {
 template <int MODE>
 hipError_t launch_batch_tiles_mode(const RasterParams* items, const ShadeParams* sitems, const BatchLists& bl,
                                    uint32_t raster_grid, uint32_t tiles_grid, int tile_size, hipStream_t s,
-                                   bool raster) {
+                                   bool raster, bool drop) {
     uint32_t* tiles_cov = bl.part_cov + raster_grid;
 #define RZ_LAUNCH(TS, B)                                                                                          \
-    if (raster)                                                                                                   \
-        hipLaunchKernelGGL((k_raster_shade_batch<TS, B, MODE>), dim3(raster_grid), dim3(B), 0, s, items, sitems, bl); \
+    if (raster && drop)                                                                                           \
+        hipLaunchKernelGGL((k_raster_shade_batch<TS, B, MODE, true>), dim3(raster_grid), dim3(B), 0, s, items,        \
+                           sitems, bl);                                                                           \
+    else if (raster)                                                                                              \
+        hipLaunchKernelGGL((k_raster_shade_batch<TS, B, MODE, false>), dim3(raster_grid), dim3(B), 0, s, items,       \
+                           sitems, bl);                                                                           \
     else                                                                                                          \
         hipLaunchKernelGGL((k_shade_tiles_batch<TS, B, MODE>), dim3(tiles_grid), dim3(B), 0, s, items, sitems, bl,    \
                            tiles_cov);
@@ -2523,12 +2540,14 @@ hipError_t launch_batch_tiles_mode(const RasterParams* items, const ShadeParams*
 // The batch's raster pass (raster = true) or its overflow shade; grids are multiples of 8.
 hipError_t launch_batch_tiles(const RasterParams* items, const ShadeParams* sitems, const BatchLists& bl,
                               uint32_t raster_grid, uint32_t tiles_grid, int tile_size, int mode, hipStream_t s,
-                              bool raster) {
+                              bool raster, bool drop) {
     switch (mode) {
         case kShadePlain:
-            return launch_batch_tiles_mode<kShadePlain>(items, sitems, bl, raster_grid, tiles_grid, tile_size, s, raster);
+            return launch_batch_tiles_mode<kShadePlain>(items, sitems, bl, raster_grid, tiles_grid, tile_size, s, raster,
+                                                         drop);
         case kShadeMlp:
-            return launch_batch_tiles_mode<kShadeMlp>(items, sitems, bl, raster_grid, tiles_grid, tile_size, s, raster);
+            return launch_batch_tiles_mode<kShadeMlp>(items, sitems, bl, raster_grid, tiles_grid, tile_size, s, raster,
+                                                         drop);
         default: return hipErrorInvalidValue;
     }
 }
