@@ -1002,8 +1002,11 @@ __device__ __forceinline__ bool fragment_key_rcp(float pxf, float pyf, float x0,
 // for D, and the quotients add u each: s <= 8.55 u P (S + 2) / |area| + 2 u, with P the
 // perimeter (bounded by |dx| + |dy| sums) and S the larger of D and the extent.  12 for 8.55
 // covers the hardware reciprocal and the roundings of the bound; 8 u the other terms.
-// Slivers (s above 1/16), areas outside [2^-40, 2^40], infinite and NaN depths have none
-// (a NaN depth never passes the depth test).
+// Those bounds are relative: a product z_i b_i below 2^-126 rounds by up to 2^-150 whatever
+// its size, so depths all below 2^-100 have no bound (above, 8 u |z|max is 2^-121 or more),
+// unless all are 0, where every depth is 0 exactly.  Slivers (s above 1/16), areas outside
+// [2^-40, 2^40], infinite and NaN depths have none either (a NaN depth never passes the
+// depth test).
 __device__ __forceinline__ float depth_floor(const float4& a, const float4& b, const float4& c, float X0, float X1,
                                                 float Y0, float Y1) {
     const float vx0 = fminf(fminf(a.x, b.x), c.x), vx1 = fmaxf(fmaxf(a.x, b.x), c.x);
@@ -1018,7 +1021,7 @@ __device__ __forceinline__ float depth_floor(const float4& a, const float4& b, c
     const float z = zmin - zabs * e;
     // (comparisons false for NaN)
     const bool ok = (S <= 1048576.0f) & (area >= 0x1p-40f) & (area <= 0x1p40f) & (e <= 0.0625f) &
-                    (fabsf(z) <= 3.4028235e38f);
+                    (fabsf(z) <= 3.4028235e38f) & ((zabs >= 0x1p-100f) | (zabs == 0.0f));
     return ok ? z : -INFINITY;
 }
 

@@ -119,6 +119,32 @@ def test_hidden_candidates_dropped(ctx, n, W, H, tuning):
         mesh.close()
 
 
+@pytest.mark.parametrize("tile", [8, 16, 32])
+@pytest.mark.parametrize("largest", [2.0 ** -149, 2.0 ** -140, 2.0 ** -131, 2.0 ** -126, 2.0 ** -101, 2.0 ** -99])
+def test_hidden_candidates_dropped_subnormal_depths(ctx, tile, largest):
+    """Depths so small that the products with the barycentric weights round by absolute, not
+    relative, amounts (a face flat at the smallest subnormal computes 0 where its weights are
+    below one half): no face may be taken to lie behind what it ties with.  Frames and batches
+    drawn without statistics equal the oracle's."""
+    scene, args = overdraw_scene(1500, 90, 70, 11)
+    rng = np.random.default_rng(12)
+    z = np.where(rng.random((1500, 1)) < 0.5, rng.choice([0.0, -0.0, 1.0, 0.5], (1500, 1)), rng.uniform(-0.2, 1, (1500, 3)))
+    scene.vertices[:, 2] = (np.broadcast_to(z, (1500, 3)) * largest).astype(np.float32).ravel()
+    ref = oracle.draw_frame(scene, args)
+    mesh = ctx.upload(scene)
+    outs = (ctx.empty((3, 70, 90), np.uint8), ctx.empty((70, 90), np.float32), ctx.empty((70, 90), np.int32))
+    try:
+        _assert_frame(_draw_plain(ctx, mesh, scene, args, None, tuning=(tile, 0)), ref, f"frame {tile} {largest}")
+        ctx.set_tuning(tile, 0)
+        ctx.draw_batch([(mesh, scene.lights_copy(), args, *outs)])
+        _assert_frame([b.download() for b in outs], ref, f"batch {tile} {largest}")
+    finally:
+        ctx.set_tuning(16, 0)
+        mesh.close()
+        for b in outs:
+            b.close()
+
+
 def test_hidden_candidates_dropped_wide_frame_and_batch(ctx):
     """The same with 64-thread workgroups (a frame of 16,384 tiles) and in a batch, as five
     launches and as one."""
