@@ -412,6 +412,13 @@ rz_status rz_copy_device(rz_ctx* ctx, void* dst_device, const void* src_device, 
 rz_status rz_check_quotients(rz_ctx* ctx, uint64_t samples, uint32_t seed, uint64_t* compared,
                              uint64_t* mismatches);
 
+/* No counterpart in the reference.  Which variants of its kernels a frame of the mesh takes
+ * under args (without statistics; tile_size 8, 16 or 32): variants[0] 1 if its raster pass
+ * drops hidden candidates, variants[1] the workgroups per block of faces of the bin pass
+ * that takes large faces by windows of tiles, 0 if it takes the other.  They differ in time,
+ * not in results.  Host only: needs no device. */
+rz_status rz_frame_variants(const rz_mesh_desc* desc, const rz_args* args, int32_t tile_size, int32_t variants[2]);
+
 /* ---- host helpers -------------------------------------------------------------- */
 
 /* Reference defaults of Args (arguments.cpp:20-31) for a width x height image, plus

@@ -78,6 +78,19 @@ struct DevBuf {
 
 }  // namespace
 
+// What frame_fit needs of a mesh.
+struct MeshExtent {
+    double face_area = 0.0;                // the mean face's (model units, pixels)
+    double layers = 0.0;                   // model space: depth complexity over the mesh's box
+    double centre[3] = {0.0, 0.0, 0.0};    // model space: the centroid
+    // Raster space, per pixel of the screen rectangle the faces cover, by winding (the front
+    // ones of wind_clockwise = 0 and 1): their area, their boxes' areas and half perimeters,
+    // and their number.
+    struct Cover {
+        double area = 0.0, box = 0.0, edges = 0.0, faces = 0.0;
+    } cover[2];
+};
+
 struct rz_mesh {
     int device = 0;
     int32_t nv = 0, nn = 0, nt = 0, nf = 0, nm = 0;
@@ -96,7 +109,7 @@ struct rz_mesh {
     // from here and the bin pass gathers nothing (uniform = 1)
     int32_t uniform = 0, uniform_n = 0, uniform_t = -1, uniform_m = 0;
     float uniform_nrm[3] = {0.f, 0.f, 0.f};   // model-space normal uniform_n
-    double layers = 0.0;                      // mesh_layers
+    MeshExtent extent;
     DevMaterial* mats = nullptr;
     uint32_t* texels = nullptr;
     float* luts = nullptr;
@@ -495,8 +508,18 @@ FrameLayout layout_batch_sync(const rz_mesh* mesh, const rz_args& a, int ts, int
     return L;
 }
 
+// How a frame draws a mesh: which raster and bin variants pay for it.  Only the time depends
+// on this, never a result.  The measurements are of both variants of each kernel on this card,
+// over screen-space and model-space triangles of 1.4 to 55,000 pixels seen 1 to 800 times over
+// at 400x400 to 2400x2400, and icospheres of 320 to 327,680 faces at 512x512 to 3840x2160.
+struct FrameFit {
+    bool overdrawn = false;    // RasterParams::overdrawn
+    uint32_t bin_parts = 0;    // BinParams::parts
+};
+
 // One frame's kernel parameters, built on the host before anything is enqueued.
 struct FrameLaunch {
+    FrameFit fit;
     CountParams cp;   // batches
     BinParams bp;
     RasterParams rp;
@@ -520,39 +543,87 @@ rz_status check_frame(rz_ctx* ctx, const rz_mesh* mesh, const rz_light* lights, 
         return fail(ctx, RZ_ERR_INVALID_ARG, "image %ux%u not in [1,%u]^2", W, H, kMaxImageSide);
     if (args->flat && mesh->raster_space)
         return fail(ctx, RZ_ERR_INVALID_ARG, "flat shading needs model-space positions");
-    if (mesh->device != ctx->device) return fail(ctx, RZ_ERR_INVALID_ARG, "mesh lives on another device");
+    if (ctx && mesh->device != ctx->device) return fail(ctx, RZ_ERR_INVALID_ARG, "mesh lives on another device");
     return RZ_OK;
 }
 
-// RasterParams::overdrawn: faces covering their extent (mesh_layers) more often than this.
-// Their raster launch is the variant that drops hidden candidates: 191 -> 77 us for 3,000
-// screen-sized triangles at 1024x1024.  A closed surface has about half its box's area (a
-// sphere: 0.52) and hides next to nothing: that variant's code and registers cost such a
-// frame more than they save (1080p icosphere raster+shade 18.0 -> 19.0 us).
-constexpr double kOverdrawn = 2.0;
-
-// BinParams::parts.  Faces are binned by windows where one, drawn to fill the frame with the
-// others, meets kWideFace tiles or more: elsewhere the few that do are not worth that
-// launch's larger code (1080p icosphere frame, a fifth of a tile a face, 0.2-0.4 us; the
-// 4M-triangle frame 0.7%).  Where binning would occupy a quarter of the CUs or less, up to 16
-// workgroups share a block's windows.  (3,000 screen-sized triangles at 1024x1024: bin pass
-// 382 us by atomics, 199 by windows in one part, 37 in 16; a 960-face sphere at 512x512,
-// half a tile a face, 9.7 by atomics and 11.1 in 16 parts.)
-constexpr double kWideFace = 2.0;
-uint32_t frame_bin_parts(int32_t nf, double layers, int32_t ntiles) {
-    const uint32_t b = frame_bin_blocks(nf);
-    if (b == 0 || layers * ntiles < kWideFace * nf) return 0;
-    return b > 64 ? 1u : std::min(512u / b, 16u);
+// RasterParams::overdrawn, from the layers of faces seen over one another, the pixels of the
+// mean one and the faces a tile holds.  Dropping costs each face a depth bound and the launch
+// its larger code (5 to 12% of a raster pass that drops nothing), and saves candidates once a
+// tile's nearest faces have covered it: it needs layers (the more, the smaller the faces: a
+// face of a few pixels costs its staging whether its candidates are dropped or not) and faces
+// enough in a tile.  In model space, where neighbouring pixels of a face lie at similar depths,
+// it gains from about 5 layers on.  Cube-filling triangles, raster+shade pass: 5.3 layers of 62
+// pixels 14.8 -> 14.4 us, of 28 pixels 15.0 -> 15.2; 13.5 layers of 102 pixels 30.1 -> 18.3, of
+// 4 pixels 53.2 -> 58.1.  Raster-space triangles with a depth of its own at each corner hide
+// less.  At 1024x1024: 3 layers of 118 pixels 29.9 -> 32.8 us, 8 layers 46.3 -> 45.4, 12 layers
+// 58.1 -> 51.8; 10 layers of 35,000 pixels (23 faces a tile) 43.1 -> 43.3, 13 layers (31) 50.1
+// -> 42.8; 3,000 screen-sized ones 169.7 -> 70.9; at 1500x1500 800 of them, 5 layers (33 faces a
+// tile), the frame 132.7 -> 121.5.  At 400x400: 10 layers of 30 pixels 19.2 -> 19.6, 20 of 7.5
+// pixels 41.4 -> 44.7.
+bool drops_hidden(bool raster_space, double layers, double pixels, double tile_faces) {
+    const double cover = pixels * layers * layers;
+    return raster_space ? pixels >= 16.0 && cover * layers >= 30000.0 && tile_faces >= 30.0
+                        : layers >= 4.5 && cover >= 1200.0 && tile_faces >= 18.0;
 }
 
-// Builds matrices and light directions (written back to `lights`, as drawing.cpp:238
-// does) and fills every pass's parameters over the working buffers `buf`.
+// BinParams::parts.  A face of 17 tiles or more else costs its wave an atomic round trip per 64
+// tiles, while the windows' larger code costs the others 2 to 10% of the pass: by windows where
+// the mean face meets 9.3 tiles (raster space) or, seen face on at the centroid, covers seven
+// quarters of one.  Bin pass, atomics -> windows: icospheres at 1080p of 1,280 faces (496
+// pixels a face) 62.7 -> 20.7 us, at 0.6 of that size 11.0 -> 11.3; cube-filling triangles at
+// 1024x1024 of 460 pixels face on 16.1 -> 14.5 (20,000 of them), of 204 pixels 11.0 -> 11.7;
+// raster-space triangles at 1024x1024 meeting 8.6 tiles 13.8 -> 14.0, 24 tiles 31.7 -> 22.6.
+// Up to 16 workgroups share a block's windows where there are few blocks; larger images have
+// more windows to share.  1,024 against 2,048 workgroups in all: 20,000 triangles of 810
+// pixels at 1024x1024 18.3 and 19.7 us (21.2 by atomics), 72,000 of 1,900 at 2400x2400 79.3 and
+// 58.4 (73.8); 3,000 screen-sized ones at 1024x1024 382 by atomics, 199 in one part, 37 in 16.
+uint32_t frame_bin_parts(int32_t nf, bool wide, double tiles) {
+    const uint32_t b = frame_bin_blocks(nf);
+    if (b == 0 || !wide) return 0;
+    return std::max(1u, std::min((tiles < 8192.0 ? 1024u : 2048u) / b, 16u));
+}
+
+FrameFit frame_fit(const rz_mesh* mesh, const rz_args& a, const rz_matrices& mats, int ts) {
+    FrameFit fit;
+    const MeshExtent& e = mesh->extent;
+    const double W = a.image_width, H = a.image_height, tile = (double)ts * ts;
+    double pixels = e.face_area, layers, tile_faces;
+    bool wide;
+    if (mesh->raster_space) {
+        const MeshExtent::Cover &c = e.cover[a.wind_clockwise ? 1 : 0], &o = e.cover[a.wind_clockwise ? 0 : 1];
+        layers = c.area;
+        tile_faces = c.box + c.edges * ts + c.faces * tile;
+        const double all = c.faces + o.faces;
+        wide = ((c.box + o.box) / tile + (c.edges + o.edges) / ts + all) > 9.3 * all;
+    } else {
+        // at the centroid's eye distance; a face at random angles shows half its area, and its
+        // box is about 1.45 times the square root of that a side (less what hangs over the image)
+        const float* m = mats.modelview;
+        const double w = std::max(-(m[2] * e.centre[0] + m[6] * e.centre[1] + m[10] * e.centre[2] + m[14]),
+                                  (double)std::fabs(a.z_near));
+        const double th = std::tan(0.5 * 0.01745329251994329576923690768489 * a.fovy_degrees);
+        const double face_on = pixels * a.scale * a.scale * W * H / (4.0 * a.aspect_ratio * th * th * w * w);
+        pixels = 0.5 * face_on;
+        layers = e.layers;
+        const double image = std::sqrt(W * H), full = 1.45 * std::sqrt(pixels);
+        const double side = full < image ? full - 0.25 * full * full / image : 0.75 * image;
+        tile_faces = layers * tile / pixels * (side / ts + 1.0) * (side / ts + 1.0);
+        wide = face_on >= 1.75 * tile;
+    }
+    // (all comparisons false for NaN: the plain variants)
+    fit.overdrawn = drops_hidden(mesh->raster_space, layers, pixels, tile_faces);
+    fit.bin_parts = frame_bin_parts(mesh->nf, wide, W * H / tile);
+    return fit;
+}
+
+// Builds the light directions (written back to `lights`, as drawing.cpp:238 does) and fills
+// every pass's parameters over the working buffers `buf`; mats: build_matrices' of `a`.
 // Single frames use generation `gen` of the counter lines (and zero the other one).
-void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args& a, uint32_t flags,
-                const FrameLayout& lay, void* const buf[kNumBufs], FrameLaunch& L, int gen = 0) {
+void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args& a, const rz_matrices& mats,
+                const FrameFit& fit, uint32_t flags, const FrameLayout& lay, void* const buf[kNumBufs],
+                FrameLaunch& L, int gen = 0) {
     const bool cleared = (flags & RZ_FLAG_CLEARED) != 0;
-    rz_matrices mats;
-    build_matrices(a, mats);
     L.lay = lay;
     std::memset(&L.sp, 0, sizeof L.sp);
     L.ext_lights.assign(nl > kMaxLights ? 6 * (size_t)(nl - kMaxLights) : 0, 0.0f);
@@ -592,7 +663,7 @@ void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args
     bp.part_front = part + lay.off_front;
     bp.part_pairs = part + lay.off_pairs;
     bp.nf = mesh->nf; bp.W = lay.W; bp.H = lay.H;
-    bp.parts = frame_bin_parts(mesh->nf, mesh->layers, lay.ntiles);
+    bp.parts = fit.bin_parts;
     bp.tiles_x = lay.tiles_x; bp.ts_log2 = lay.tsl; bp.cap = lay.cap;
     bp.wind_cw = a.wind_clockwise != 0;
     bp.ntiles = lay.ntiles;
@@ -628,7 +699,7 @@ void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args
     rp.ovf_list = bp.ovf_list;
     rp.front_mask = bp.front_mask;
     rp.face_v = mesh->bin_face_v;
-    rp.overdrawn = mesh->layers > kOverdrawn ? 1 : 0;
+    rp.overdrawn = fit.overdrawn ? 1 : 0;
     rp.max_blocks = lay.raster_grid;
     L.orp = rp;   // batches: k_overflow_batch
     L.orp.part_frag = part + lay.off_ovf;
@@ -693,14 +764,15 @@ int frame_bin_cap(const rz_ctx* ctx, const rz_mesh* mesh, uint32_t ntiles) {
 // tiles than resident workgroups, 64-thread workgroups keep four times as many tiles
 // in flight (1080p: 23 against 63 us; 4M triangles at 4096x4096: 326 against 254 us)
 // flags: the frame's; without RZ_FLAG_CLEARED the raster pass stages the input depths
-// in dynamic LDS, which the residency count includes.
-void frame_shape(const rz_ctx* ctx, const rz_mesh* mesh, const rz_args& a, int mode, uint32_t flags, uint32_t& ntiles, bool& narrow,
-                 uint32_t& grid) {
+// in dynamic LDS, which the residency count includes.  drop: the variant that drops hidden
+// candidates.
+void frame_shape(const rz_ctx* ctx, const rz_args& a, bool drop, int mode, uint32_t flags, uint32_t& ntiles,
+                 bool& narrow, uint32_t& grid) {
     ntiles = ((a.image_width + ctx->tile_size - 1) / ctx->tile_size) *
              ((a.image_height + ctx->tile_size - 1) / ctx->tile_size);
     narrow = ctx->tile_size == 16 && ntiles >= kNarrowTiles;
     const uint32_t per_cu =
-        raster_blocks_per_cu(ctx->tile_size, ctx->fused, mode, narrow, (flags & RZ_FLAG_CLEARED) == 0, mesh->layers > kOverdrawn);
+        raster_blocks_per_cu(ctx->tile_size, ctx->fused, mode, narrow, (flags & RZ_FLAG_CLEARED) == 0, drop);
     grid = (uint32_t)ctx->cus * per_cu / 8u * 8u;
     if (grid < 8) grid = 8;
 }
@@ -720,16 +792,21 @@ rz_status stage_ext_lights(rz_ctx* ctx, DevBuf& buf, FrameLaunch& L, bool stales
 }
 
 // Single frame: validates, sizes the context's working buffers and fills L.  mode: the
-// shading mode (-1: the one flags select).
+// shading mode (-1: the one flags select).  like: a frame prepared before whose variants this
+// one takes too (the frames of a graph: the variants decide the launch's size and so the
+// statistics', and no later frame may grow a buffer that an earlier one already points into).
 rz_status prepare_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args* args,
-                        uint32_t flags, FrameLaunch& L, int gen, int mode = -1) {
+                        uint32_t flags, FrameLaunch& L, int gen, int mode = -1, const FrameLaunch* like = nullptr) {
     rz_status st = check_frame(ctx, mesh, lights, nl, args);
     if (st != RZ_OK) return st;
     RZ_HIP(ctx, hipSetDevice(ctx->device));
     if (mode < 0) mode = (flags & RZ_FLAG_MLP_SHADE) ? kShadeMlp : kShadePlain;
+    rz_matrices mats;
+    build_matrices(*args, mats);
+    L.fit = like ? like->fit : frame_fit(mesh, *args, mats, ctx->tile_size);
     uint32_t ntiles = 0, grid = 0;
     bool narrow = false;
-    frame_shape(ctx, mesh, *args, mode, flags, ntiles, narrow, grid);
+    frame_shape(ctx, *args, L.fit.overdrawn, mode, flags, ntiles, narrow, grid);
     const int cap = frame_bin_cap(ctx, mesh, ntiles);
     const bool can_overflow = (uint32_t)cap < (uint32_t)mesh->nf;
     const FrameLayout lay = layout_frame(mesh, *args, ctx->tile_size, cap, ctx->fused, grid,
@@ -743,7 +820,7 @@ rz_status prepare_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
     for (int i = 0; i < kNumBufs; ++i) ptrs[i] = bufs[i]->ptr;
     if ((flags & RZ_FLAG_MLP_SHADE) && !ctx->mlp_ready)
         return fail(ctx, RZ_ERR_INVALID_ARG, "RZ_FLAG_MLP_SHADE without network weights (rz_mlp_init / rz_mlp_set_weights)");
-    fill_frame(mesh, lights, nl, *args, flags, lay, ptrs, L, gen);
+    fill_frame(mesh, lights, nl, *args, mats, L.fit, flags, lay, ptrs, L, gen);
     if ((st = stage_ext_lights(ctx, ctx->lights_ext, L, false)) != RZ_OK) return st;
     L.rp.narrow = narrow ? 1 : 0;
     L.sp.mode = mode;
@@ -928,6 +1005,23 @@ constexpr size_t kSyncWords = 3 * 8 * (kCountStride / 2);
 constexpr size_t kCursorWord = kSyncWords + 16;   // (64-bit words from the block's start)
 constexpr size_t kSyncBytes = (kCursorWord + 16) * 8;
 
+// Checks a batch's items; the raster pass drops hidden candidates unless statistics are asked for.
+rz_status batch_fit(rz_ctx* ctx, const rz_batch_item* items, int32_t n, bool stats, std::vector<rz_matrices>& mats,
+                    std::vector<FrameFit>& fits, bool& drop) {
+    mats.resize(n);
+    fits.resize(n);
+    for (int32_t i = 0; i < n; ++i) {
+        const rz_batch_item& it = items[i];
+        rz_status st = check_frame(ctx, it.mesh, it.lights, it.num_lights, &it.args);
+        if (st != RZ_OK) return st;
+        if (!it.frame || !it.depth) return fail(ctx, RZ_ERR_INVALID_ARG, "batch item %d: null frame or depth", i);
+        build_matrices(it.args, mats[i]);
+        fits[i] = frame_fit(it.mesh, it.args, mats[i], ctx->tile_size);
+    }
+    drop = !stats;
+    return RZ_OK;
+}
+
 rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32_t flags, bool stats,
                         DevBuf& arena, DevBuf& tables, BatchLaunch& B) {
     if (n < 1 || !items) return fail(ctx, RZ_ERR_INVALID_ARG, "empty batch");
@@ -941,7 +1035,10 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
     B.ts = ctx->tile_size;
     B.mode = (flags & RZ_FLAG_MLP_SHADE) ? kShadeMlp : kShadePlain;
     B.persistent = false;
-    B.drop = !stats;
+    std::vector<rz_matrices> mats;
+    std::vector<FrameFit> fits;
+    rz_status st = batch_fit(ctx, items, n, stats, mats, fits, B.drop);
+    if (st != RZ_OK) return st;
     const int bblock = 256;
     uint32_t grid = (uint32_t)ctx->cus * raster_batch_blocks_per_cu(B.ts, B.mode, B.drop) / 8u * 8u;
     B.raster_grid = grid < 8 ? 8 : grid;
@@ -953,9 +1050,6 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
     size_t stat_bytes = batch_stat_bytes, work_bytes = 0, stride = 0;
     for (int32_t i = 0; i < n; ++i) {
         const rz_batch_item& it = items[i];
-        rz_status st = check_frame(ctx, it.mesh, it.lights, it.num_lights, &it.args);
-        if (st != RZ_OK) return st;
-        if (!it.frame || !it.depth) return fail(ctx, RZ_ERR_INVALID_ARG, "batch item %d: null frame or depth", i);
         lays[i] = layout_frame(it.mesh, it.args, ctx->tile_size, ctx->bin_cap > 0 ? ctx->bin_cap : kDefaultBinCap,
                                true, 0, 0, true, bblock);
         if ((uint32_t)lays[i].ntiles > kListTileMask)
@@ -965,8 +1059,7 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
         stride += (size_t)lays[i].ntiles;
     }
     const size_t list_bytes = align256(9 * stride * 4);   // 8 lists, then the overflowed tiles
-    rz_status st = ensure(ctx, arena, stat_bytes + list_bytes + work_bytes);
-    if (st != RZ_OK) return st;
+    if ((st = ensure(ctx, arena, stat_bytes + list_bytes + work_bytes)) != RZ_OK) return st;
     B.frames.assign(n, FrameLaunch());
     B.faces.assign(n, 0);
     B.arena_part_bytes = stat_bytes;
@@ -988,7 +1081,7 @@ rz_status prepare_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
         ptrs[kBufPart] = base + so;
         so += align256(lays[i].bytes[kBufPart]);
         FrameLaunch& L = B.frames[i];
-        fill_frame(it.mesh, it.lights, it.num_lights, it.args, flags, lays[i], ptrs, L);
+        fill_frame(it.mesh, it.lights, it.num_lights, it.args, mats[i], fits[i], flags, lays[i], ptrs, L);
         L.sp.mlp = (const uint16_t*)ctx->mlp_packed.ptr;
         bind_outputs(L, cleared, it.frame, it.depth, it.ids);
         // the shared lists; their 8 counters are the first mesh's (cleared by the first launch)
@@ -1092,7 +1185,10 @@ rz_status prepare_batch_sync(rz_ctx* ctx, const rz_batch_item* items, int32_t n,
     B.ts = ctx->tile_size;
     B.mode = (flags & RZ_FLAG_MLP_SHADE) ? kShadeMlp : kShadePlain;
     B.persistent = true;
-    B.drop = !stats;
+    std::vector<rz_matrices> mats;
+    std::vector<FrameFit> fits;
+    rz_status st = batch_fit(ctx, items, n, stats, mats, fits, B.drop);
+    if (st != RZ_OK) return st;
     const int bblock = batch_block(B.ts);
     // every workgroup of the launch resident at once: the launch's occupancy on every CU
     uint32_t grid = (uint32_t)ctx->cus * batch_frame_blocks_per_cu(B.ts, B.mode, B.drop) / 8u * 8u;
@@ -1105,9 +1201,6 @@ rz_status prepare_batch_sync(rz_ctx* ctx, const rz_batch_item* items, int32_t n,
     size_t stat_bytes = batch_stat_bytes, work_bytes = 0, stride = 0;
     for (int32_t i = 0; i < n; ++i) {
         const rz_batch_item& it = items[i];
-        rz_status st = check_frame(ctx, it.mesh, it.lights, it.num_lights, &it.args);
-        if (st != RZ_OK) return st;
-        if (!it.frame || !it.depth) return fail(ctx, RZ_ERR_INVALID_ARG, "batch item %d: null frame or depth", i);
         lays[i] = layout_batch_sync(it.mesh, it.args, B.ts, cap, bblock);
         if ((uint32_t)lays[i].ntiles > kListTileMask)
             return fail(ctx, RZ_ERR_INVALID_ARG, "batch item %d: %d tiles, at most %u", i, lays[i].ntiles, kListTileMask);
@@ -1117,8 +1210,7 @@ rz_status prepare_batch_sync(rz_ctx* ctx, const rz_batch_item* items, int32_t n,
         stride += (size_t)lays[i].ntiles;
     }
     const size_t list_bytes = align256(9 * stride * 4);   // 8 lists, then the overflowed tiles
-    rz_status st = ensure(ctx, arena, stat_bytes + list_bytes + work_bytes);
-    if (st != RZ_OK) return st;
+    if ((st = ensure(ctx, arena, stat_bytes + list_bytes + work_bytes)) != RZ_OK) return st;
     B.frames.assign(n, FrameLaunch());
     B.frames1.assign(n, FrameLaunch());
     B.faces.assign(n, 0);
@@ -1141,7 +1233,7 @@ rz_status prepare_batch_sync(rz_ctx* ctx, const rz_batch_item* items, int32_t n,
         so += align256(lays[i].bytes[kBufPart]);
         for (int g = 0; g < 2; ++g) {
             FrameLaunch& L = g ? B.frames1[i] : B.frames[i];
-            fill_frame(it.mesh, it.lights, it.num_lights, it.args, flags, lays[i], ptrs, L, g);
+            fill_frame(it.mesh, it.lights, it.num_lights, it.args, mats[i], fits[i], flags, lays[i], ptrs, L, g);
             L.sp.mlp = (const uint16_t*)ctx->mlp_packed.ptr;
             L.sp.mode = B.mode;
             bind_outputs(L, cleared, it.frame, it.depth, it.ids);
@@ -1600,39 +1692,116 @@ void bin_faces(const rz_mesh_desc* d, std::vector<BinFace>& out) {
     }
 }
 
-// How many times the faces cover their extent: their total area over the surface of the box
-// their centroids spread over (model space), or over its screen rectangle (raster space).  Seen from anywhere, front faces show about a quarter
-// of the area and the box a quarter of its surface, so the ratio is about the depth
-// complexity over the box: 0.5 for a sphere, tens for triangle soups.  (A side of the box:
-// the uniform distribution's 2 sqrt(3) standard deviations, which a few far vertices barely
-// move.)
-double mesh_layers(const rz_mesh_desc* d) {
-    const int stride = d->raster_space ? 4 : 3, dims = d->raster_space ? 2 : 3;
-    double area = 0.0, sum[3] = {0, 0, 0}, sq[3] = {0, 0, 0};
+// Model space: layers is the faces' total area over the surface of the box their centroids
+// spread over (seen from anywhere, front faces show about a quarter of the area and the box a
+// quarter of its surface, so the ratio is about the depth complexity over the box: 0.5 for a
+// sphere, tens for triangle soups).  A side of the box is the uniform distribution's
+// 2 sqrt(3) standard deviations, which a few far vertices barely move.
+void model_extent(const rz_mesh_desc* d, MeshExtent& e) {
+    double area = 0.0, sum[3] = {0, 0, 0}, sq[3] = {0, 0, 0}, side[3];
     for (int32_t f = 0; f < d->num_faces; ++f) {
         const float* v[3];
-        for (int k = 0; k < 3; ++k) v[k] = d->vertices + (size_t)stride * d->faces[f].vertices[k];
-        double e[3] = {0, 0, 0}, g[3] = {0, 0, 0};
-        for (int c = 0; c < dims; ++c) {
-            e[c] = (double)v[1][c] - v[0][c];
-            g[c] = (double)v[2][c] - v[0][c];
-            const double m = ((double)v[0][c] + v[1][c] + v[2][c]) / 3.0;
-            sum[c] += m;
-            sq[c] += m * m;
+        for (int k = 0; k < 3; ++k) v[k] = d->vertices + (size_t)3 * d->faces[f].vertices[k];
+        double p[3], q[3];
+        for (int c = 0; c < 3; ++c) {
+            p[c] = (double)v[1][c] - v[0][c];
+            q[c] = (double)v[2][c] - v[0][c];
+            const double t = ((double)v[0][c] + v[1][c] + v[2][c]) / 3.0;
+            sum[c] += t;
+            sq[c] += t * t;
         }
-        const double x = e[1] * g[2] - e[2] * g[1], y = e[2] * g[0] - e[0] * g[2], z = e[0] * g[1] - e[1] * g[0];
+        const double x = p[1] * q[2] - p[2] * q[1], y = p[2] * q[0] - p[0] * q[2], z = p[0] * q[1] - p[1] * q[0];
         area += 0.5 * std::sqrt(x * x + y * y + z * z);
     }
-    double side[3] = {0, 0, 0};
     const double n = d->num_faces > 0 ? (double)d->num_faces : 1.0;
-    for (int c = 0; c < dims; ++c) side[c] = std::sqrt(12.0 * std::max(0.0, sq[c] / n - (sum[c] / n) * (sum[c] / n)));
-    const double box = d->raster_space ? side[0] * side[1]
-                                       : 2.0 * (side[0] * side[1] + side[1] * side[2] + side[2] * side[0]);
-    const double r = area / box;   // (infinite for faces around one point)
-    return r > 0.0 ? r : 0.0;      // (NaN: 0)
+    for (int c = 0; c < 3; ++c) {
+        e.centre[c] = sum[c] / n;
+        side[c] = std::sqrt(12.0 * std::max(0.0, sq[c] / n - e.centre[c] * e.centre[c]));
+    }
+    e.face_area = area / n;
+    e.layers = area / (2.0 * (side[0] * side[1] + side[1] * side[2] + side[2] * side[0]));
+}
+
+// Raster space, from at most 32,768 of the faces: the screen rectangle is twice the middle half
+// of their centroids on each axis, from 0 on, and what hangs over it is not seen (a face's area
+// by its box's share).
+void raster_extent(const rz_mesh_desc* d, MeshExtent& e) {
+    const int32_t step = std::max(1, d->num_faces / 16384);
+    struct Box {
+        double lo[2], hi[2], z;
+    };
+    std::vector<Box> boxes;
+    std::vector<double> mid[2];
+    for (int32_t f = 0; f < d->num_faces; f += step) {
+        const float* v[3];
+        for (int k = 0; k < 3; ++k) v[k] = d->vertices + (size_t)4 * d->faces[f].vertices[k];
+        Box b;
+        for (int c = 0; c < 2; ++c) {
+            b.lo[c] = std::min(std::min(v[0][c], v[1][c]), v[2][c]);
+            b.hi[c] = std::max(std::max(v[0][c], v[1][c]), v[2][c]);
+        }
+        // (signed_area is -z / 2: front where it is positive, or not with wind_clockwise)
+        b.z = ((double)v[1][0] - v[0][0]) * ((double)v[2][1] - v[0][1]) -
+              ((double)v[1][1] - v[0][1]) * ((double)v[2][0] - v[0][0]);
+        const double x = ((double)v[0][0] + v[1][0] + v[2][0]) / 3.0, y = ((double)v[0][1] + v[1][1] + v[2][1]) / 3.0;
+        if (!std::isfinite(b.z) || !std::isfinite(x) || !std::isfinite(y)) continue;
+        boxes.push_back(b);
+        mid[0].push_back(x);
+        mid[1].push_back(y);
+    }
+    if (boxes.empty()) return;
+    double lo[2], hi[2];
+    const size_t n = boxes.size();
+    for (int c = 0; c < 2; ++c) {
+        std::nth_element(mid[c].begin(), mid[c].begin() + n / 4, mid[c].end());
+        const double q1 = mid[c][n / 4];
+        std::nth_element(mid[c].begin(), mid[c].begin() + 3 * n / 4, mid[c].end());
+        const double q3 = mid[c][3 * n / 4];
+        lo[c] = std::max(0.0, 0.5 * (q1 + q3) - (q3 - q1));
+        hi[c] = 0.5 * (q1 + q3) + (q3 - q1);
+    }
+    const double per_pixel = (double)step / ((hi[0] - lo[0]) * (hi[1] - lo[1]));
+    double total = 0.0;
+    for (const Box& b : boxes) {
+        MeshExtent::Cover& c = e.cover[b.z >= 0.0 ? 1 : 0];
+        c.faces += per_pixel;
+        const double w = std::min(b.hi[0], hi[0]) - std::max(b.lo[0], lo[0]);
+        const double h = std::min(b.hi[1], hi[1]) - std::max(b.lo[1], lo[1]);
+        if (!(w > 0.0 && h > 0.0)) continue;
+        const double area = 0.5 * std::fabs(b.z) * (w * h) / ((b.hi[0] - b.lo[0]) * (b.hi[1] - b.lo[1]));
+        total += area;
+        c.area += area * per_pixel;
+        c.box += w * h * per_pixel;
+        c.edges += (w + h) * per_pixel;
+    }
+    e.face_area = total / (double)n;
+}
+
+void mesh_extent(const rz_mesh_desc* d, MeshExtent& e) {
+    if (d->raster_space)
+        raster_extent(d, e);
+    else
+        model_extent(d, e);
 }
 
 }  // namespace
+
+rz_status rz_frame_variants(const rz_mesh_desc* d, const rz_args* args, int32_t tile_size, int32_t variants[2]) {
+    if (!args || !variants || (tile_size != 8 && tile_size != 16 && tile_size != 32)) return RZ_ERR_INVALID_ARG;
+    rz_status st = validate_mesh(nullptr, d);
+    if (st != RZ_OK) return st;
+    rz_mesh m;
+    m.nf = d->num_faces;
+    m.raster_space = d->raster_space != 0;
+    if ((st = check_frame(nullptr, &m, nullptr, 0, args)) != RZ_OK) return st;
+    mesh_extent(d, m.extent);
+    rz_matrices mats;
+    build_matrices(*args, mats);
+    const FrameFit fit = frame_fit(&m, *args, mats, tile_size);
+    variants[0] = fit.overdrawn ? 1 : 0;
+    variants[1] = (int32_t)fit.bin_parts;
+    return RZ_OK;
+}
 
 rz_status rz_mesh_create(rz_ctx* ctx, const rz_mesh_desc* d, rz_mesh** out) {
     if (!ctx || !out) return RZ_ERR_INVALID_ARG;
@@ -1648,7 +1817,7 @@ rz_status rz_mesh_create(rz_ctx* ctx, const rz_mesh_desc* d, rz_mesh** out) {
     m->nf = d->num_faces;
     m->nm = d->num_materials;
     m->raster_space = d->raster_space != 0;
-    m->layers = mesh_layers(d);
+    mesh_extent(d, m->extent);
     auto cleanup = [&](rz_status s) {
         rz_mesh_destroy(ctx, m);
         return s;
@@ -1991,7 +2160,8 @@ rz_status rz_graph_create(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, in
     rz_args a = args ? *args : rz_args{};
     // frame k uses generation k % 2 of the counter lines (rz_graph_launch readies 0)
     for (int32_t k = 0; k < frames; ++k) {
-        rz_status st = prepare_frame(ctx, mesh, lights, nl, args ? &a : nullptr, flags, launches[k], k & 1);
+        rz_status st = prepare_frame(ctx, mesh, lights, nl, args ? &a : nullptr, flags, launches[k], k & 1, -1,
+                                     k > 0 ? &launches[0] : nullptr);
         if (st != RZ_OK) return st;
         bind_outputs(launches[k], (flags & RZ_FLAG_CLEARED) != 0, frame_d, depth_d, ids_d);
         a.tait_bryan_angles[1] += ry_step;   // the spin loop's rotation about y (renderer.cpp:124)
@@ -2533,9 +2703,12 @@ rz_status rz_draw_frame_noalloc(rz_ctx* ctx, const rz_mesh* mesh, rz_light* ligh
     rz_status st = check_frame(ctx, mesh, lights, nl, args);
     if (st != RZ_OK) return st;
     RZ_HIP(ctx, hipSetDevice(ctx->device));
+    rz_matrices mats;
+    build_matrices(*args, mats);
+    const FrameFit fit = frame_fit(mesh, *args, mats, ctx->tile_size);
     uint32_t ntiles = 0, grid = 0;
     bool narrow = false;
-    frame_shape(ctx, mesh, *args, kShadePlain, flags, ntiles, narrow, grid);
+    frame_shape(ctx, *args, fit.overdrawn, kShadePlain, flags, ntiles, narrow, grid);
     // Working set in `scratch`: the layout of rz_draw_frame with a bin capacity that fits.
     // With the fused pipeline and room for every face in every bin no tile can overflow
     // and the visibility buffer is never touched, so it takes no space.
@@ -2573,7 +2746,7 @@ rz_status rz_draw_frame_noalloc(rz_ctx* ctx, const rz_mesh* mesh, rz_light* ligh
         at += align256(lay.bytes[b]);
     }
     FrameLaunch L;
-    fill_frame(mesh, lights, nl, *args, flags, lay, ptrs, L, 0);
+    fill_frame(mesh, lights, nl, *args, mats, fit, flags, lay, ptrs, L, 0);
     L.rp.narrow = narrow ? 1 : 0;
     L.sp.max_blocks = lay.tiles_grid;
     bind_outputs(L, (flags & RZ_FLAG_CLEARED) != 0, frame_device, depth_device, id_device);

@@ -168,12 +168,12 @@ struct RasterParams {
     int32_t ts_log2;
     uint32_t cap;
     uint32_t max_blocks;        // workgroups of the list-driven launch (a multiple of 8)
-    // The mesh's faces cover its extent several times over: the raster pass that drops hidden
-    // candidates (raster_body).  For a mesh seen about once a pixel that variant's larger code
-    // and register need cost more than the little it drops (1080p icosphere 18.0 -> 19.0 us,
-    // 4M-triangle frame 141.3 -> 143.4 us), while 3,000 screen-sized triangles went 191 ->
-    // 77 us.  0 where statistics are asked for: every inside-test fragment is then counted.
-    // (Batches: their launch decides.)
+    // The raster pass that drops hidden candidates (raster_body), for meshes whose faces lie
+    // several times over one another on the screen (frame_fit).  For a mesh seen about once a
+    // pixel that variant's larger code and register need cost more than the little it drops
+    // (1080p icosphere 18.0 -> 19.0 us, 4M-triangle frame 141.3 -> 143.4 us), while 3,000
+    // screen-sized triangles went 191 -> 77 us.  0 where statistics are asked for: every
+    // inside-test fragment is then counted.  (Batches: their launch decides.)
     int32_t overdrawn;
     int32_t narrow;             // 16-pixel tiles by 64-thread workgroups (frames with many tiles)
     int32_t pre_cleared;        // outputs cleared by the bin launch

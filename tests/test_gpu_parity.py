@@ -180,6 +180,45 @@ def test_hidden_candidates_dropped_wide_frame_and_batch(ctx):
                 b.close()
 
 
+def test_turning_mesh_whose_size_on_screen_changes(ctx):
+    """A dense cloud of triangles off the axis it turns about: far away at first, near at the
+    end, so that an eager frame's choice of kernel variants changes on the way.  Every frame of
+    a graph and of a spin loop equals the eager frame's and the oracle's."""
+    rng = np.random.default_rng(5)
+    n = 4000
+    c = np.array([0.0, 0.0, -1.9]) + rng.uniform(-0.3, 0.3, (n, 1, 3))
+    pos = (c + rng.uniform(-0.2, 0.2, (n, 3, 3))).reshape(-1, 3).astype(np.float32)
+    tri = np.arange(3 * n).reshape(n, 3)
+    scene = Scene(pos, np.array([[0.0, 0.0, 1.0]], np.float32), np.zeros((1, 2), np.float32),
+                  make_faces(tri, n=np.zeros_like(tri), t=None), [MaterialSpec((0.9, 0.8, 0.7))],
+                  make_lights([[0.0, 0.0, -1.0]], [200.0 * np.pi], [[1.0, 0.9, 0.8]]))
+    W, H, frames = 320, 240, 4
+    step = float(np.float32(np.pi / (frames - 1)))
+    mesh = ctx.upload(scene)
+    f, d = ctx.empty((3, H, W), np.uint8), ctx.empty((H, W), np.float32)
+    try:
+        angles = [np.float32(0.0)]
+        for _ in range(frames - 1):
+            angles.append(np.float32(angles[-1] + np.float32(step)))
+        spin = ctx.spin(mesh, scene.lights_copy(), make_args(W, H), f.ptr, d.ptr)
+        for k, ry in enumerate(angles):
+            args = make_args(W, H, angles=(0.0, float(ry), 0.0))
+            ref = oracle.draw_frame(scene, args)
+            graph = ctx.graph(mesh, scene.lights_copy(), make_args(W, H), f.ptr, d.ptr, k + 1, ry_step=step)
+            for draw in (lambda: ctx.draw_device(mesh, scene.lights_copy(), args, f.ptr, d.ptr), graph.launch,
+                         lambda: spin.frame((0.0, float(ry), 0.0))):
+                draw()
+                ctx.sync()
+                got = f.download(), d.download()
+                assert np.array_equal(got[1].view(np.uint32), ref[1].view(np.uint32)), k
+                assert np.array_equal(got[0], ref[0]), k
+            graph.close()
+        spin.close()
+    finally:
+        for x in (mesh, f, d):
+            x.close()
+
+
 @pytest.mark.parametrize("tile,cap", [(8, 0), (16, 0), (32, 0), (16, 5)])
 @pytest.mark.parametrize("wide,tiny", [(1, 0), (40, 0), (300, 200), (6, 9000)])
 def test_faces_meeting_many_tiles(ctx, wide, tiny, tile, cap):
