@@ -180,6 +180,30 @@ def test_hidden_candidates_dropped_wide_frame_and_batch(ctx):
                 b.close()
 
 
+@pytest.mark.parametrize("closed,dense", [(4, 0), (4, 1), (1, 3), (0, 2)])
+def test_batch_of_closed_and_overdrawn_meshes(ctx, closed, dense):
+    """Batches that hide nothing, a little and most of what they draw, without statistics (their
+    raster pass drops hidden candidates where that pays for the whole batch): frames, depths
+    and ids equal the oracle's."""
+    work = [scenes.icosphere_scene(seed=k, width=150 + 20 * k, height=130, subdivisions=3, texture_size=16) for k in range(closed)]
+    work += [overdraw_scene(1500, 110, 90, k) for k in range(dense)]
+    meshes = [ctx.upload(s) for s, _ in work]
+    outs = [tuple(ctx.empty(sh, t) for sh, t in (((3, a.image_height, a.image_width), np.uint8),
+                                                 ((a.image_height, a.image_width), np.float32),
+                                                 ((a.image_height, a.image_width), np.int32))) for _, a in work]
+    batch = [(m, s.lights_copy(), a, *o) for m, (s, a), o in zip(meshes, work, outs)]
+    try:
+        for persistent in (False, True):
+            ctx.set_batch_persistent(persistent)
+            ctx.draw_batch(batch)
+            for k, (o, (s, a)) in enumerate(zip(outs, work)):
+                _assert_frame([b.download() for b in o], oracle.draw_frame(s, a), f"item {k} persistent {persistent}")
+    finally:
+        ctx.set_batch_persistent(False)
+        for x in (*meshes, *(b for o in outs for b in o)):
+            x.close()
+
+
 def test_turning_mesh_whose_size_on_screen_changes(ctx):
     """A dense cloud of triangles off the axis it turns about: far away at first, near at the
     end, so that an eager frame's choice of kernel variants changes on the way.  Every frame of
