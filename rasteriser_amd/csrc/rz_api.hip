@@ -5,6 +5,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -278,7 +279,19 @@ rz_status download(rz_ctx* ctx, const Download* d, int count) {
         std::memcpy(t.dst, ctx->stage + (size_t)(k % kStageChunks) * kStageBytes, t.bytes);
         t.free.store(true, std::memory_order_release);
     };
-    auto help = [&] {
+    // The helpers sleep until the first chunk is here: whatever the stream still does before
+    // it (the frame, others queued) costs their cores nothing.
+    std::mutex m;
+    std::condition_variable arrived;
+    bool begun = false;
+    auto begin = [&] {
+        {
+            std::lock_guard<std::mutex> lock(m);
+            begun = true;
+        }
+        arrived.notify_all();
+    };
+    auto copy_chunks = [&] {
         for (int k; (k = claimed.fetch_add(1)) < chunks;) {
             while (ready.load(std::memory_order_acquire) <= k) {
                 if (failed.load()) return;
@@ -286,6 +299,13 @@ rz_status download(rz_ctx* ctx, const Download* d, int count) {
             }
             copy_out(k);
         }
+    };
+    auto help = [&] {
+        {
+            std::unique_lock<std::mutex> lock(m);
+            arrived.wait(lock, [&] { return begun; });
+        }
+        copy_chunks();
     };
     std::thread helper[kStageThreads - 1];
     bool helped = false;
@@ -323,12 +343,15 @@ rz_status download(rz_ctx* ctx, const Download* d, int count) {
         if (e == hipSuccess) e = hipEventSynchronize(ctx->stage_ev[k % kStageChunks]);
         if (e != hipSuccess) break;
         ready.store(k + 1, std::memory_order_release);
+        if (k == 0) begin();
         if (!helped) copy_out(claimed.fetch_add(1));
     }
-    if (e != hipSuccess)
+    if (e != hipSuccess) {
         failed.store(true);
-    else
-        help();   // (what no helper has claimed)
+        begin();   // (a helper still asleep ends too)
+    } else {
+        copy_chunks();   // (what no helper has claimed)
+    }
     for (std::thread& t : helper)
         if (t.joinable()) t.join();
     if (e != hipSuccess) {

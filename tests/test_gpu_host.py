@@ -4,6 +4,7 @@ its frame.png must equal the oracle's frame of the same scene byte for byte."""
 import ctypes as C
 import os
 import subprocess
+import time
 
 import numpy as np
 import pytest
@@ -145,6 +146,31 @@ def test_downloads_through_pinned_chunks(nbytes):
             assert np.array_equal(out[:n], data[start:]), f"{nbytes} bytes from {start}"
             assert (out[n:] == 0xA5).all()
         a.close()
+
+
+def test_download_behind_queued_work_leaves_the_cpu_alone():
+    """The threads that copy a download's chunks out sleep until the first chunk is there: a
+    download queued behind frames keeps at most the calling thread busy (it used to keep four
+    cores busy for as long as the frames took)."""
+    scene, args = scenes.large_triangle_scene(5, 3000, 1024)
+    with rz.Context(0) as c:
+        mesh = c.upload(scene)
+        f, d = c.empty((3, 1024, 1024), np.uint8), c.empty((1024, 1024), np.float32)
+        big = c.empty((8 << 20,), np.uint8)
+        graph = c.graph(mesh, scene.lights_copy(), args, f.ptr, d.ptr, 500)
+        big.download()
+        graph.launch()
+        c.sync()
+        wall, cpu = time.perf_counter(), time.process_time()
+        for _ in range(8):
+            graph.launch()
+        big.download()
+        wall, cpu = time.perf_counter() - wall, time.process_time() - cpu
+        assert wall > 0.1   # (eight times 500 frames of about 0.1 ms)
+        # the caller's own wait may spin, and the runtime's thread beside it
+        assert cpu < 2.5 * wall, (cpu, wall)
+        for x in (graph, mesh, f, d, big):
+            x.close()
 
 
 def test_download_into_pinned_memory():
