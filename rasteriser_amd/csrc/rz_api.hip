@@ -71,6 +71,10 @@ constexpr int kPersistentPerCU = 4;
 constexpr int kStageChunks = 16;
 constexpr size_t kStageBytes = (size_t)1 << 20;   // (a multiple of 16)
 constexpr int kStageThreads = 4;
+// The least bytes that go through them.  Copied by the runtime and through the chunks: 1 MiB
+// 61 and 104 us, 2 MiB 120 and 124, 3 MiB 180 and 147, 4 MiB 240 and 168, 16 MiB 945 and 440
+// (chunks of a quarter MiB: 84, 116, 155, 190 and 620).
+constexpr size_t kStageLeast = (size_t)3 << 20;
 
 struct DevBuf {
     void* ptr = nullptr;
@@ -241,7 +245,7 @@ rz_status download(rz_ctx* ctx, const Download* d, int count) {
     hipStream_t s = ctx->stream;
     size_t total = 0;
     for (int i = 0; i < count; ++i) total += d[i].bytes;
-    if (total >= 4 * kStageBytes && !ctx->stage && !ctx->stage_failed) {
+    if (total >= kStageLeast && !ctx->stage && !ctx->stage_failed) {
         void* p = nullptr;
         hipError_t e = hipHostMalloc(&p, kStageChunks * kStageBytes, hipHostMallocDefault);
         for (int i = 0; i < kStageChunks && e == hipSuccess; ++i)
@@ -254,7 +258,7 @@ rz_status download(rz_ctx* ctx, const Download* d, int count) {
             ctx->stage_failed = true;   // (events made so far go with the context)
         }
     }
-    bool staged = total >= 4 * kStageBytes && ctx->stage;
+    bool staged = total >= kStageLeast && ctx->stage;
     for (int i = 0; i < count && staged; ++i)
         staged = (uintptr_t)d[i].src % 16 == 0 && !host_pinned(d[i].dst);
     if (!staged) {
@@ -1646,7 +1650,7 @@ rz_status rz_copy_to_host(rz_ctx* ctx, void* dst, const void* src, size_t bytes)
     RZ_HIP(ctx, hipSetDevice(ctx->device));
     // (a kernel reads `src`: only where all of it is memory of this device; the runtime's
     // copy takes, or refuses, everything else)
-    if (!within_allocation(ctx, src, bytes)) {
+    if (bytes < kStageLeast || !within_allocation(ctx, src, bytes)) {
         RZ_HIP(ctx, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
         RZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
         return RZ_OK;

@@ -148,6 +148,19 @@ def test_downloads_through_pinned_chunks(nbytes):
         a.close()
 
 
+@pytest.mark.parametrize("nbytes", [(3 << 20) - 1, 3 << 20, (3 << 20) + 1])
+def test_downloads_around_the_staged_size(nbytes):
+    """The last size the runtime copies and the first ones that go through pinned chunks."""
+    data = np.random.default_rng(nbytes).integers(0, 256, nbytes, dtype=np.uint8)
+    with rz.Context(0) as c:
+        a = c.empty((nbytes,), np.uint8)
+        a.upload(data)
+        out = np.full(nbytes + 64, 0xA5, np.uint8)
+        assert c.lib.rz_copy_to_host(c.handle, out.ctypes.data, C.c_void_p(a.ptr), nbytes) == 0
+        assert np.array_equal(out[:nbytes], data) and (out[nbytes:] == 0xA5).all()
+        a.close()
+
+
 def test_download_behind_queued_work_leaves_the_cpu_alone():
     """The threads that copy a download's chunks out sleep until the first chunk is there: a
     download queued behind frames keeps at most the calling thread busy (it used to keep four
