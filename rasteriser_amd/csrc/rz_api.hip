@@ -824,8 +824,10 @@ rz_status stage_ext_lights(rz_ctx* ctx, DevBuf& buf, FrameLaunch& L, bool stales
 // shading mode (-1: the one flags select).  like: a frame prepared before whose variants this
 // one takes too (the frames of a graph: the variants decide the launch's size and so the
 // statistics', and no later frame may grow a buffer that an earlier one already points into).
+// counts: every inside-test fragment is counted, so no hidden candidate is dropped.
 rz_status prepare_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args* args,
-                        uint32_t flags, FrameLaunch& L, int gen, int mode = -1, const FrameLaunch* like = nullptr) {
+                        uint32_t flags, FrameLaunch& L, int gen, int mode = -1, const FrameLaunch* like = nullptr,
+                        bool counts = false) {
     rz_status st = check_frame(ctx, mesh, lights, nl, args);
     if (st != RZ_OK) return st;
     RZ_HIP(ctx, hipSetDevice(ctx->device));
@@ -833,6 +835,7 @@ rz_status prepare_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
     rz_matrices mats;
     build_matrices(*args, mats);
     L.fit = like ? like->fit : frame_fit(mesh, *args, mats, ctx->tile_size);
+    if (counts) L.fit.overdrawn = false;
     uint32_t ntiles = 0, grid = 0;
     bool narrow = false;
     frame_shape(ctx, *args, L.fit.overdrawn, mode, flags, ntiles, narrow, grid);
@@ -2137,7 +2140,7 @@ rz_status rz_draw_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
     const bool cleared = (flags & RZ_FLAG_CLEARED) != 0;
     const bool on_device = (flags & RZ_FLAG_DEVICE_BUFFERS) != 0;
     FrameLaunch L;
-    rz_status st = prepare_frame(ctx, mesh, lights, nl, args, flags, L, ctx->count_gen);
+    rz_status st = prepare_frame(ctx, mesh, lights, nl, args, flags, L, ctx->count_gen, -1, nullptr, stats != nullptr);
     if (st != RZ_OK) return st;
     if (!frame_buffer || !depth_buffer) return fail(ctx, RZ_ERR_INVALID_ARG, "null frame or depth buffer");
     const size_t np = L.lay.np;
@@ -2160,7 +2163,6 @@ rz_status rz_draw_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
         }
     }
     bind_outputs(L, cleared, frame_d, depth_d, ids_d);
-    if (stats) L.rp.overdrawn = 0;   // (every fragment is counted)
     if ((st = run_frame(ctx, L, ctx->profiling)) != RZ_OK) return st;
     if (!on_device) {
         const Download d[3] = {{frame_buffer, frame_d, np * 3}, {depth_buffer, depth_d, np * 4}, {id_buffer, ids_d, np * 4}};
