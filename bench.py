@@ -291,12 +291,13 @@ def batched(ctx, rz, scenes, np, frames):
             idh = i.download()
             vis += int(np.unique(idh[idh >= 0]).size)
         # per-pass times: HIP events around each launch of one batch frame of five launches
-        # (median of 5); the one-launch frame's phases as spans of the workgroups' clocks
+        # (median of 5), of the kernels a batch without statistics runs; the one-launch frame's
+        # phases as spans of the workgroups' clocks
         ctx.set_profiling(True)
         phases = {}
         for one in (False, True):
             ctx.set_batch_persistent(one)
-            runs = [ctx.draw_batch(batch, stats=True) for _ in range(5)]
+            runs = [ctx.draw_batch(batch, rz.RZ_FLAG_CLEARED | rz.RZ_FLAG_TIMES_ONLY, stats=True) for _ in range(5)]
             phases[one] = {k: float(np.median([r["ms_" + k] for r in runs])) * 1000.0
                            for k in ("vertex", "bin", "raster", "overflow", "shade", "frame")}
         ctx.set_batch_persistent(default_one)

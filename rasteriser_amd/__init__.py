@@ -13,13 +13,13 @@ import weakref
 import numpy as np
 
 from . import abi
-from .abi import (RZ_FLAG_ASYNC, RZ_FLAG_CLEARED, RZ_FLAG_DEVICE_BUFFERS, RZ_FLAG_MLP_SHADE, RZ_MLP_PARAMS,
+from .abi import (RZ_FLAG_ASYNC, RZ_FLAG_CLEARED, RZ_FLAG_DEVICE_BUFFERS, RZ_FLAG_MLP_SHADE, RZ_FLAG_TIMES_ONLY, RZ_MLP_PARAMS,
                   RZ_MLP_SAMPLE_FLOATS, Args, BatchItem, FrameStats, Matrices, make_args)
 from .scene import MaterialSpec, Scene, make_faces, make_lights
 
 __all__ = ["Context", "Mesh", "RzError", "Scene", "MaterialSpec", "make_faces", "make_lights",
            "make_args", "library_path", "load_library", "frame_matrices",
-           "RZ_FLAG_CLEARED", "RZ_FLAG_DEVICE_BUFFERS", "RZ_FLAG_ASYNC", "RZ_FLAG_MLP_SHADE",
+           "RZ_FLAG_CLEARED", "RZ_FLAG_DEVICE_BUFFERS", "RZ_FLAG_ASYNC", "RZ_FLAG_MLP_SHADE", "RZ_FLAG_TIMES_ONLY",
            "RZ_MLP_PARAMS", "RZ_MLP_SAMPLE_FLOATS"]
 
 _HERE = os.path.dirname(os.path.abspath(__file__))

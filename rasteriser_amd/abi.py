@@ -21,6 +21,7 @@ RZ_FLAG_CLEARED = 1
 RZ_FLAG_DEVICE_BUFFERS = 2
 RZ_FLAG_ASYNC = 4
 RZ_FLAG_MLP_SHADE = 8
+RZ_FLAG_TIMES_ONLY = 16
 
 RZ_MLP_PARAMS = 5187
 RZ_MLP_SAMPLE_FLOATS = 15

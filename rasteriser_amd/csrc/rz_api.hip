@@ -2139,8 +2139,9 @@ rz_status rz_draw_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
     if (!ctx) return RZ_ERR_INVALID_ARG;
     const bool cleared = (flags & RZ_FLAG_CLEARED) != 0;
     const bool on_device = (flags & RZ_FLAG_DEVICE_BUFFERS) != 0;
+    const bool counts = stats && !(flags & RZ_FLAG_TIMES_ONLY);
     FrameLaunch L;
-    rz_status st = prepare_frame(ctx, mesh, lights, nl, args, flags, L, ctx->count_gen, -1, nullptr, stats != nullptr);
+    rz_status st = prepare_frame(ctx, mesh, lights, nl, args, flags, L, ctx->count_gen, -1, nullptr, counts);
     if (st != RZ_OK) return st;
     if (!frame_buffer || !depth_buffer) return fail(ctx, RZ_ERR_INVALID_ARG, "null frame or depth buffer");
     const size_t np = L.lay.np;
@@ -2169,7 +2170,7 @@ rz_status rz_draw_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
         if ((st = download(ctx, d, id_buffer ? 3 : 2)) != RZ_OK) return st;
     }
     std::vector<uint32_t> list_counts, lists;
-    if (stats) {
+    if (counts) {
         RZ_HIP(ctx, hipMemcpyAsync(ctx->host_counters, L.counters, kNumCounters * 8, hipMemcpyDeviceToHost, s));
         ctx->host_partials.resize(L.lay.n_part);
         RZ_HIP(ctx, hipMemcpyAsync(ctx->host_partials.data(), L.part, L.lay.n_part * 4, hipMemcpyDeviceToHost, s));
@@ -2181,9 +2182,11 @@ rz_status rz_draw_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
     if (stats || !on_device || !(flags & RZ_FLAG_ASYNC)) RZ_HIP(ctx, hipStreamSynchronize(s));
     if (stats) {
         std::memset(stats, 0, sizeof *stats);
-        reduce_stats(L, ctx->host_counters, ctx->host_partials.data(), (uint64_t)mesh->nf, stats);
-        count_listed(list_counts.data(), lists.data(), (size_t)L.lay.ntiles, &L.lay, 1, false, &stats->raster_tiles,
-                     &stats->raster_pixels);
+        if (counts) {
+            reduce_stats(L, ctx->host_counters, ctx->host_partials.data(), (uint64_t)mesh->nf, stats);
+            count_listed(list_counts.data(), lists.data(), (size_t)L.lay.ntiles, &L.lay, 1, false,
+                         &stats->raster_tiles, &stats->raster_pixels);
+        }
         if (ctx->profiling && (st = event_times(ctx, stats)) != RZ_OK) return st;
     }
     return RZ_OK;
@@ -2474,8 +2477,9 @@ void rz_graph_destroy(rz_graph* g) {
 
 rz_status rz_draw_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint32_t flags, rz_frame_stats* stats) {
     if (!ctx) return RZ_ERR_INVALID_ARG;
+    const bool counts = stats && !(flags & RZ_FLAG_TIMES_ONLY);
     BatchLaunch B;
-    rz_status st = prepare_any_batch(ctx, items, n, flags, stats != nullptr, ctx->batch_arena, ctx->batch_tables, B);
+    rz_status st = prepare_any_batch(ctx, items, n, flags, counts, ctx->batch_arena, ctx->batch_tables, B);
     if (st != RZ_OK) return st;
     const bool phase_clock = ctx->profiling && B.persistent;
     if (phase_clock) {
@@ -2489,29 +2493,30 @@ rz_status rz_draw_batch(rz_ctx* ctx, const rz_batch_item* items, int32_t n, uint
         RZ_HIP(ctx, hipMemcpy(B.q.clock, init, sizeof init, hipMemcpyHostToDevice));
     }
     if ((st = enqueue_batch(ctx, B, ctx->stream, ctx->profiling)) != RZ_OK) return st;
-    if (stats) {
+    if (counts) {
         if ((st = batch_stats(ctx, B, ctx->batch_arena, stats)) != RZ_OK) return st;
-        if (ctx->profiling) {
-            if (phase_clock) {
-                // each phase as the span of its work (first start to last end: the phases
-                // of different workgroups overlap around the barriers)
-                unsigned long long clk[8];
-                RZ_HIP(ctx, hipMemcpy(clk, B.q.clock, sizeof clk, hipMemcpyDeviceToHost));
-                float* ms[4] = {&stats->ms_bin, &stats->ms_raster, &stats->ms_overflow, &stats->ms_shade};
-                stats->ms_vertex = 0.0f;   // (the bin work transforms each face's corners)
-                for (int k = 0; k < 4; ++k)
-                    *ms[k] = clk[2 * k + 1] > clk[2 * k] ? (float)(clk[2 * k + 1] - clk[2 * k]) * 1e-5f : 0.0f;
-                RZ_HIP(ctx, hipEventElapsedTime(&stats->ms_frame, ctx->ev[0], ctx->ev[5]));
-            } else if ((st = event_times(ctx, stats)) != RZ_OK) {
-                return st;
-            }
-        }
-    } else if (!(flags & RZ_FLAG_ASYNC)) {
+    } else if (stats || !(flags & RZ_FLAG_ASYNC)) {
         RZ_HIP(ctx, hipStreamSynchronize(ctx->stream));
         if (B.persistent) {
             uint32_t err = 0;
             RZ_HIP(ctx, hipMemcpy(&err, B.q.error, 4, hipMemcpyDeviceToHost));
             if (err) return fail(ctx, RZ_ERR_HIP, "batch frame: a barrier wait gave up");
+        }
+        if (stats) std::memset(stats, 0, sizeof *stats);
+    }
+    if (stats && ctx->profiling) {
+        if (phase_clock) {
+            // each phase as the span of its work (first start to last end: the phases
+            // of different workgroups overlap around the barriers)
+            unsigned long long clk[8];
+            RZ_HIP(ctx, hipMemcpy(clk, B.q.clock, sizeof clk, hipMemcpyDeviceToHost));
+            float* ms[4] = {&stats->ms_bin, &stats->ms_raster, &stats->ms_overflow, &stats->ms_shade};
+            stats->ms_vertex = 0.0f;   // (the bin work transforms each face's corners)
+            for (int k = 0; k < 4; ++k)
+                *ms[k] = clk[2 * k + 1] > clk[2 * k] ? (float)(clk[2 * k + 1] - clk[2 * k]) * 1e-5f : 0.0f;
+            RZ_HIP(ctx, hipEventElapsedTime(&stats->ms_frame, ctx->ev[0], ctx->ev[5]));
+        } else if ((st = event_times(ctx, stats)) != RZ_OK) {
+            return st;
         }
     }
     return RZ_OK;

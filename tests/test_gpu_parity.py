@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import oracle
+import rasteriser_amd as rz
 from rasteriser_amd import MaterialSpec, Scene, make_args, make_faces, make_lights, scenes
 from tests.parity import check
 
@@ -201,6 +202,50 @@ def test_batch_of_closed_and_overdrawn_meshes(ctx, closed, dense):
     finally:
         ctx.set_batch_persistent(False)
         for x in (*meshes, *(b for o in outs for b in o)):
+            x.close()
+
+
+def test_pass_times_of_a_frame_as_drawn_without_statistics(ctx):
+    """RZ_FLAG_TIMES_ONLY: the times of the raster variant that plain calls run (it drops hidden
+    candidates; on these triangles the counting one takes more than twice as long), no counts,
+    and the frame itself, for single frames and batches of either form."""
+    scene, args = scenes.large_triangle_scene(n=3000)
+    H, W = args.image_height, args.image_width
+    ref = oracle.draw_frame(scene, args)
+    mesh = ctx.upload(scene)
+    f, d = ctx.empty((3, H, W), np.uint8), ctx.empty((H, W), np.float32)
+    batch = [(mesh, scene.lights_copy(), args, f, d, None)]
+    flags = rz.RZ_FLAG_CLEARED
+
+    def raster_ms(draw, flags):
+        ms = []
+        for _ in range(5):
+            st = draw(flags)
+            ms.append(st["ms_raster"])
+        assert np.array_equal(d.download().view(np.uint32), ref[1].view(np.uint32))
+        assert np.array_equal(f.download(), ref[0])
+        counts = [st[k] for k in ("triangles", "front_triangles", "bin_pairs", "fragments", "covered_pixels", "raster_tiles")]
+        assert all(c > 0 for c in counts) if not flags & rz.RZ_FLAG_TIMES_ONLY else not any(counts)
+        assert st["ms_frame"] > 0
+        return float(np.median(ms))
+
+    ctx.set_profiling(True)
+    try:
+        for persistent in (None, False, True):
+            ctx.set_batch_persistent(bool(persistent))
+            draw = (lambda fl: ctx.draw_device(mesh, scene.lights_copy(), args, f.ptr, d.ptr, flags=fl, stats=True)) \
+                if persistent is None else (lambda fl: ctx.draw_batch(batch, fl, stats=True))
+            counted, plain = raster_ms(draw, flags), raster_ms(draw, flags | rz.RZ_FLAG_TIMES_ONLY)
+            assert plain > 0
+            if not persistent:   # (the one launch's phases are spans, which overlap)
+                assert plain < 0.75 * counted, (persistent, plain, counted)
+        ctx.set_profiling(False)
+        st = ctx.draw_device(mesh, scene.lights_copy(), args, f.ptr, d.ptr, flags=flags | rz.RZ_FLAG_TIMES_ONLY, stats=True)
+        assert not any(st.values())
+    finally:
+        ctx.set_profiling(False)
+        ctx.set_batch_persistent(False)
+        for x in (mesh, f, d):
             x.close()
 
 
