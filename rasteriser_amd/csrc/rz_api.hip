@@ -2042,9 +2042,13 @@ rz_status rz_time_passes(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int
         return fail(ctx, RZ_ERR_INVALID_ARG, "rz_time_passes: device buffers, reps >= 1 and RZ_FLAG_CLEARED required");
     if ((flags & RZ_FLAG_MLP_SHADE) && !ctx->mlp_ready)
         return fail(ctx, RZ_ERR_INVALID_ARG, "RZ_FLAG_MLP_SHADE without network weights");
+    // (the chain frame's launch, prepared below, may be the larger one: its buffers are sized
+    // first, so that no pointer of the others is left behind by a buffer that grows)
+    FrameLaunch Lc;
+    rz_status st = prepare_frame(ctx, mesh, lights, nl, args, flags, Lc, 0, kShadeChain);
+    if (st != RZ_OK) return st;
     // the frame with each generation of counter lines (the bin launches alternate)
     FrameLaunch L2[2];
-    rz_status st = RZ_OK;
     for (int g = 0; g < 2; ++g) {
         if ((st = prepare_frame(ctx, mesh, lights, nl, args, flags, L2[g], g)) != RZ_OK) return st;
         bind_outputs(L2[g], true, frame_device, depth_device, nullptr);
@@ -2090,7 +2094,6 @@ rz_status rz_time_passes(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int
     const FrameLaunch& L = L2[gen];
     if ((st = run_frame(ctx, L, false)) != RZ_OK) return st;
     // the same frame's shading with neither light loop nor network (kShadeChain)
-    FrameLaunch Lc;
     if ((st = prepare_frame(ctx, mesh, lights, nl, args, flags, Lc, gen, kShadeChain)) != RZ_OK) return st;
     bind_outputs(Lc, true, frame_device, depth_device, nullptr);
     auto raster = [&](int32_t, hipStream_t cs) -> rz_status {

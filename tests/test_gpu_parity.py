@@ -205,6 +205,27 @@ def test_batch_of_closed_and_overdrawn_meshes(ctx, closed, dense):
             x.close()
 
 
+@pytest.mark.parametrize("tile,flags", [(16, 0), (32, 0), (16, rz.RZ_FLAG_MLP_SHADE), (32, rz.RZ_FLAG_MLP_SHADE)])
+def test_time_passes_first_on_a_context(tile, flags):
+    """Timing as a context's first call: the shading chain's launch may be larger than the
+    frame's, and every launch must use the buffers as they are once both are prepared.  The
+    frame it leaves is the plain one's."""
+    scene, args = overdraw_scene(4000, 333, 250, 4000)
+    with rz.Context(0) as c:
+        c.set_tuning(tile, 0)
+        c.mlp_init(1)
+        mesh = c.upload(scene)
+        f, d = c.empty((3, 250, 333), np.uint8), c.empty((250, 333), np.float32)
+        us = c.time_passes(mesh, scene.lights_copy(), args, f, d, reps=3, flags=flags)
+        assert us["raster"] > 0 and us["chain"] > 0
+        got = f.download(), d.download()
+        c.draw_device(mesh, scene.lights_copy(), args, f.ptr, d.ptr, flags=flags | rz.RZ_FLAG_CLEARED)
+        assert np.array_equal(got[0], f.download())
+        assert np.array_equal(got[1].view(np.uint32), oracle.draw_frame(scene, args)[1].view(np.uint32))
+        for x in (mesh, f, d):
+            x.close()
+
+
 def test_pass_times_of_a_frame_as_drawn_without_statistics(ctx):
     """RZ_FLAG_TIMES_ONLY: the times of the raster variant that plain calls run (it drops hidden
     candidates; on these triangles the counting one takes more than twice as long), no counts,
