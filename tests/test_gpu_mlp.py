@@ -111,6 +111,88 @@ def test_training_step_over_chunks(ctx, n, batch):
     assert agree.mean() > 0.995, agree.mean()
 
 
+def _grad_and_spread(p, rows):
+    """The gradient over the rows, and per parameter the mean size of its samples' terms."""
+    X, T = rows[:, :M.N_IN], rows[:, M.N_IN:]
+    g = M.loss_and_grad(p, X, T)[1]
+    W1, b1, W2, b2, W3, b3 = M.unpack(p)
+    r = M._rounder(True)
+    w2, w3 = r(W2), r(W3)
+    a1 = r(X) @ r(W1).T + b1
+    h1 = r(np.maximum(a1, 0))
+    a2 = h1 @ w2.T + b2
+    h2 = r(np.maximum(a2, 0))
+    dy = np.abs(2.0 * (h2 @ w3.T + b3 - T) / len(X))
+    d2 = (dy @ np.abs(w3)) * (a2 > 0)
+    d1 = (d2 @ np.abs(w2)) * (a1 > 0)
+    parts = d1.T @ np.abs(r(X)), d1.sum(0), d2.T @ h1, d2.sum(0), dy.T @ h2, dy.sum(0)
+    return g, np.concatenate([q.ravel() for q in parts])
+
+
+def _second_adam_step(ga, gb):
+    """The second Adam update (learning rate 1) after a first one of gradient ga."""
+    m, v = 0.09 * ga + 0.1 * gb, 0.000999 * ga * ga + 0.001 * gb * gb
+    return -(m / (1 - 0.9 ** 2)) / (np.sqrt(v / (1 - 0.999 ** 2)) + 1e-8)
+
+
+@pytest.mark.parametrize("chunks", [259, 512, 1027])
+def test_gradient_over_chunks_by_value(ctx, chunks):
+    """The summed gradient of a step whose workgroups take several chunks, every parameter of
+    every block by value.  A step's update is invariant to its gradient's size, so a first step
+    of 64 samples with learning rate 0 sets the moments and the second one's update shows the
+    ratio of the two gradients.  The samples that a workgroup's first, second, ... and last
+    chunks draw have targets scaled so that each of these groups makes up a like share of the
+    gradient: a group lost, taken twice or mixed up moves most updates (checked with the numpy
+    gradient)."""
+    seed, n = 33, 1 << 18
+    p = M.random_params(16, scale=0.5)
+    rng = np.random.default_rng(chunks)
+    data = np.concatenate([rng.uniform(-1, 1, (n, M.N_IN)), rng.uniform(0, 1, (n, M.N_OUT))], 1).astype(np.float32)
+    rows_a, rows_b = _drawn(n, 64, 1, seed), _drawn(n, 64 * chunks, 2, seed)
+    group = (np.arange(64 * chunks) // 64) // 256          # a workgroup's chunk number
+    groups = int(group[-1]) + 1
+    for k in range(groups):                                # (later groups overwrite shared rows: still known data)
+        data[rows_b[group == k], M.N_IN:] *= np.float32(256.0 * 64 / (group == k).sum())
+    ctx.mlp_set_weights(p)
+    buf = ctx.empty(data.shape, np.float32)
+    try:
+        buf.upload(data)
+        ctx.mlp_train(buf, n, steps=1, batch=64, lr=0.0, seed=seed)
+        assert np.array_equal(ctx.mlp_get_weights(), p)
+        ctx.mlp_train(buf, n, steps=1, batch=64 * chunks, lr=1.0, seed=seed)
+        got = ctx.mlp_get_weights().astype(np.float64) - p.astype(np.float64)
+    finally:
+        buf.close()
+    (ga, sa), (gb, sb) = _grad_and_spread(p, data[rows_a]), _grad_and_spread(p, data[rows_b])
+    # Each gradient to 1e-3 of its terms' mean size: sums of 64 products, five chunks and 16 + 16
+    # partials in f32 stay below 400 2^-24 of it, and of 64 samples a few activations may round
+    # to bf16 the other way (3 / 64 of 2^-8).  The update's own f32 arithmetic: 5e-5 of it (1 -
+    # 0.999^2 cancels all but 2e-3, half of that error through the root), and 2e-6 for the
+    # subtraction from a weight of up to 1.
+    ends = [_second_adam_step(ga + i * 1e-3 * sa, gb + j * 1e-3 * sb) for i in (-1, 0, 1) for j in (-1, 0, 1)]
+    slack = 2e-6 + 5e-5 * np.abs(ends[4])
+    lo, hi = np.minimum.reduce(ends) - slack, np.maximum.reduce(ends) + slack
+    narrow = (hi - lo < 0.05) & (sb > 0) & (sa > 0)
+
+    def misses(update, block):
+        o = sel[block] & narrow
+        return np.mean((update[o] < lo[o]) | (update[o] > hi[o])), o.sum()
+
+    sel, at = {}, 0
+    for name, size in (("W1", 768), ("b1", 64), ("W2", 4096), ("b2", 64), ("W3", 192), ("b3", 3)):
+        sel[name] = np.zeros(M.N_PARAMS, bool)
+        sel[name][at:at + size] = True
+        at += size
+    for name in sel:
+        miss, count = misses(got, name)
+        assert count >= 0.5 * (sel[name] & (sb > 0) & (sa > 0)).sum(), (name, count)
+        assert miss <= 0.002, (name, miss, count)
+    for k in range(groups):   # the same check of a gradient without one of the groups fails
+        gl = _grad_and_spread(p, data[rows_b[group != k]])[0] * (group != k).mean()
+        for name in ("W1", "W2", "W3"):
+            assert misses(_second_adam_step(ga, gl), name)[0] > 0.5, (name, k)
+
+
 def test_collect_train_and_shade(ctx):
     scene, args = scenes.learned_shading_scene(width=320, height=180, subdivisions=4, map_size=128)
     mesh = ctx.upload(scene)
