@@ -1,5 +1,7 @@
 """GPU parity of the frame path: librz (through its C ABI) against the CPU oracle on
 the same seeded inputs.  Face ids, depth bits and colour bytes must match exactly."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -179,6 +181,44 @@ def test_hidden_candidates_dropped_wide_frame_and_batch(ctx):
         for o in outs:
             for b in o:
                 b.close()
+
+
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("given", [False, True])
+def test_hidden_candidates_dropped_one_wave_of_several_chunks(ctx, given, fused):
+    """16-pixel tiles by 64-thread workgroups (16,512 tiles, the last of each row and column cut
+    by the image's edge) with several chunks of 64 faces in a tile: those after the first drop
+    faces behind the tile's farthest pixel.  Flat faces that tie, -0 and 0, infinite and NaN
+    depths, a cleared and a given depth buffer: equal to the oracle's."""
+    scene, _ = scenes.large_triangle_scene(3, 6000, 2048)
+    W, H = 2041, 2063
+    args = make_args(W, H)
+    rng = np.random.default_rng(8)
+    z = scene.vertices[:, 2].reshape(-1, 3).copy()
+    flat = rng.random(len(z)) < 0.4
+    z[flat] = rng.choice([-0.0, 0.0, -0.5, 0.25, 0.25 + 2.0 ** -24, 0.5, 0.75], (flat.sum(), 1))
+    bad = rng.random(len(z)) < 0.02
+    z[bad, rng.integers(0, 3, bad.sum())] = rng.choice([np.inf, -np.inf, np.nan], bad.sum())
+    scene.vertices[:, 2] = z.ravel()
+    # that the frame reaches what this is about: the variant, and some three chunks in a tile
+    desc, keep = scene.desc()
+    out = (C.c_int32 * 2)()
+    assert rz.load_library().rz_frame_variants(C.byref(desc), C.byref(args), 16, out) == 0 and out[0] == 1
+    del keep
+    assert (-(-W // 16)) * (-(-H // 16)) >= 16384
+    depth = frame = None
+    if given:
+        depth = rng.uniform(-0.3, 1.0, (H, W)).astype(np.float32)
+        depth[::7, ::5] = 0.25
+        frame = np.full((3, H, W), 7, np.uint8)
+    ref = oracle.draw_frame(scene, args, frame=frame, depth=depth)
+    mesh = ctx.upload(scene)
+    try:
+        _, _, _, st = ctx.draw(mesh, scene.lights_copy(), args, stats=True)
+        assert st["bin_pairs"] / st["raster_tiles"] > 150
+        _assert_frame(_draw_plain(ctx, mesh, scene, args, depth, fused), ref, f"given {given} fused {fused}")
+    finally:
+        mesh.close()
 
 
 @pytest.mark.parametrize("closed,dense", [(4, 0), (4, 1), (1, 3), (0, 2)])
