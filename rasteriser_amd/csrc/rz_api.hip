@@ -1766,8 +1766,9 @@ void model_extent(const rz_mesh_desc* d, MeshExtent& e) {
 }
 
 // Raster space, from at most 32,768 of the faces: the screen rectangle is twice the middle half
-// of their centroids on each axis, from 0 on, and what hangs over it is not seen (a face's area
-// by its box's share).
+// of their centroids on each axis, or for a handful of faces, or centroids in a line, what
+// their boxes cover; from 0 on, and what hangs over it is not seen (a face's area by its box's
+// share).
 void raster_extent(const rz_mesh_desc* d, MeshExtent& e) {
     const int32_t step = std::max(1, d->num_faces / 16384);
     struct Box {
@@ -1802,6 +1803,14 @@ void raster_extent(const rz_mesh_desc* d, MeshExtent& e) {
         const double q3 = mid[c][3 * n / 4];
         lo[c] = std::max(0.0, 0.5 * (q1 + q3) - (q3 - q1));
         hi[c] = 0.5 * (q1 + q3) + (q3 - q1);
+    }
+    for (int c = 0; c < 2; ++c) {
+        if (n >= 16 && hi[c] > lo[c]) continue;
+        lo[c] = hi[c] = std::max(0.0, boxes[0].lo[c]);
+        for (const Box& b : boxes) {
+            lo[c] = std::min(lo[c], std::max(0.0, b.lo[c]));
+            hi[c] = std::max(hi[c], b.hi[c]);
+        }
     }
     const double per_pixel = (double)step / ((hi[0] - lo[0]) * (hi[1] - lo[1]));
     double total = 0.0;

@@ -75,6 +75,23 @@ def test_screen_sized_triangles(n, size, drop):
     assert variants(*scenes.large_triangle_scene(5, n, size)) == (drop, 16)
 
 
+@pytest.mark.parametrize("copies", [1, 2, 40])
+@pytest.mark.parametrize("shape", ["triangle", "quad", "strip"])
+def test_screen_filling_shapes(shape, copies):
+    """A handful of faces, or many in one place: their centroids span no rectangle, their boxes
+    do.  They meet thousands of tiles each (a single 1080p triangle's bin pass 111 us by
+    atomics, 23 by windows)."""
+    corners = {"triangle": [[(-10, -10), (-10, 2200), (3900, -10)]],
+               "quad": [[(0, 0), (0, 1080), (1920, 0)], [(1920, 0), (0, 1080), (1920, 1080)]],
+               "strip": [[(0, 500), (0, 580), (1920, 500)], [(1920, 500), (0, 580), (1920, 580)]]}[shape] * copies
+    xy = np.array(corners, np.float64)
+    n = len(xy)
+    verts = np.concatenate([xy, np.full((n, 3, 1), 0.5), np.ones((n, 3, 1))], 2).reshape(-1, 4).astype(np.float32)
+    scene = _scene(verts, np.arange(3 * n).reshape(n, 3), True)
+    drop, parts = variants(scene, make_args(1920, 1080))
+    assert parts == 16 and drop == (copies == 40)
+
+
 def test_front_faces_alone_count():
     """One winding only: seen or culled by wind_clockwise."""
     scene, args = triangles(_n(12, 1024, 64), 1024, 64)
