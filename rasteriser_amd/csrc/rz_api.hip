@@ -1010,7 +1010,7 @@ struct BatchLaunch {
     std::vector<uint64_t> faces;
     int ts = 16;
     int mode = kShadePlain;
-    bool drop = true;               // hidden candidates dropped: no statistics asked for
+    bool drop = true;               // hidden candidates dropped (batch_fit)
     const CountParams* d_cp = nullptr;
     const BinParams* d_bp = nullptr;
     const RasterParams* d_rp = nullptr;

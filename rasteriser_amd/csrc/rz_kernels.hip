@@ -1871,8 +1871,8 @@ __global__ __launch_bounds__(256) void k_bin_batch(const BinParams* __restrict__
 // A batch's raster pass: one resident grid over the tile lists the meshes share, entry
 // (mesh << kListMeshShift) | tile, raster and shade of the tile with its mesh's
 // parameters.
-// DROP: hidden candidates are dropped (raster_body), in every batch whose caller asks for no
-// statistics.
+// DROP: hidden candidates are dropped (raster_body), in batches whose overdrawn meshes make that
+// pay (batch_fit in rz_api.hip).
 template <int TS, int BLOCK, int MODE, bool DROP>
 __global__ __launch_bounds__(BLOCK, MODE == kShadeMlp ? 3 : 6) void k_raster_shade_batch(
     const RasterParams* __restrict__ items, const ShadeParams* __restrict__ sitems, BatchLists bl) {
@@ -2331,7 +2331,7 @@ hipError_t launch_bin(const BinParams& p, hipStream_t s) {
 
 // Resident workgroups per CU of the list-driven raster kernel for this configuration.
 // depth_in: the frame stages an input depth buffer (the kernels' dynamic LDS).
-// drop: the mesh is overdrawn.
+// drop: the variant that drops hidden candidates.
 uint32_t raster_blocks_per_cu(int tile_size, bool fused, int mode, bool narrow, bool depth_in, bool drop) {
     const void* f = nullptr;
     int block = 256;
