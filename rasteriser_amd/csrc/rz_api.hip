@@ -765,6 +765,9 @@ void fill_frame(const rz_mesh* mesh, rz_light* lights, int32_t nl, const rz_args
     sp.inv_p11 = th;
 }
 
+// At most this many workgroups of any kernel are resident on a CU (32 waves).
+constexpr uint32_t kMaxBlocksPerCU = 32;
+
 // Frames with at least this many 16-pixel tiles raster them with 64-thread workgroups.
 constexpr uint32_t kNarrowTiles = 16384;
 
@@ -841,8 +844,11 @@ rz_status prepare_frame(rz_ctx* ctx, const rz_mesh* mesh, rz_light* lights, int3
     frame_shape(ctx, *args, L.fit.overdrawn, mode, flags, ntiles, narrow, grid);
     const int cap = frame_bin_cap(ctx, mesh, ntiles);
     const bool can_overflow = (uint32_t)cap < (uint32_t)mesh->nf;
-    const FrameLayout lay = layout_frame(mesh, *args, ctx->tile_size, cap, ctx->fused, grid,
-                                         can_overflow ? ctx->persistent_blocks : 0u, false);
+    FrameLayout lay = layout_frame(mesh, *args, ctx->tile_size, cap, ctx->fused, grid,
+                                   can_overflow ? ctx->persistent_blocks : 0u, false);
+    // (the statistics' room for any variant's grid: a frame of the same mesh and image must not
+    // grow a buffer that a captured one points into because it takes another variant)
+    lay.bytes[kBufPart] += (ctx->fused ? 2u : 1u) * ((size_t)ctx->cus * kMaxBlocksPerCU - grid) * 4;
     DevBuf* bufs[kNumBufs] = {&ctx->rec,   &ctx->tile_count, &ctx->bins,
                               &ctx->vis,    &ctx->lists,   &ctx->counters, &ctx->partials};
     void* ptrs[kNumBufs];

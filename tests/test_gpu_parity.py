@@ -266,6 +266,43 @@ def test_time_passes_first_on_a_context(tile, flags):
             x.close()
 
 
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("tile", [8, 16, 32])
+def test_graphs_outlive_frames_of_other_variants(tile, fused):
+    """A captured frame stays valid when its context draws the same mesh and image in other
+    ways: with counts, far away, close by, timed: no buffer grows, whichever
+    kernel variants those frames take."""
+    rng = np.random.default_rng(5)
+    pos = (rng.uniform(-0.5, 0.5, (4000, 1, 3)) + rng.uniform(-0.2, 0.2, (4000, 3, 3))).reshape(-1, 3).astype(np.float32)
+    tri = np.arange(12000).reshape(4000, 3)
+    scene = Scene(pos, np.array([[0.0, 0.0, 1.0]], np.float32), np.zeros((1, 2), np.float32),
+                  make_faces(tri, n=np.zeros_like(tri), t=None), [MaterialSpec((0.9, 0.8, 0.7))],
+                  make_lights([[0.0, 0.0, -1.0]], [200.0 * np.pi], [[1.0, 0.9, 0.8]]))
+    W = H = 300
+    with rz.Context(0) as c:
+        c.set_tuning(tile, 0)
+        c.set_fused_shade(fused)
+        mesh = c.upload(scene)
+        f, d = c.empty((3, H, W), np.uint8), c.empty((H, W), np.float32)
+        views = [make_args(W, H, scale=s) for s in (1.0, 0.01, 2.5)]
+        for first in views:
+            graph = c.graph(mesh, scene.lights_copy(), first, f.ptr, d.ptr, 2)
+            graph.launch()
+            c.sync()
+            want = f.download(), d.download()
+            c.draw_device(mesh, scene.lights_copy(), first, f.ptr, d.ptr, stats=True)
+            for other in views:
+                c.draw_device(mesh, scene.lights_copy(), other, f.ptr, d.ptr)
+            c.time_passes(mesh, scene.lights_copy(), first, f, d, reps=2)
+            graph.launch()
+            c.sync()
+            assert np.array_equal(f.download(), want[0])
+            assert np.array_equal(d.download().view(np.uint32), want[1].view(np.uint32))
+            graph.close()
+        for x in (mesh, f, d):
+            x.close()
+
+
 def test_pass_times_of_a_frame_as_drawn_without_statistics(ctx):
     """RZ_FLAG_TIMES_ONLY: the times of the raster variant that plain calls run (it drops hidden
     candidates; on these triangles the counting one takes more than twice as long), no counts,
