@@ -359,7 +359,7 @@ __device__ __forceinline__ void bin_body(const BinParams& p, int blk, unsigned c
     // The code from here on starts on a line of the instruction cache, wherever the code
     // above ends.  Left to fall where it may, its position cost up to 4% of the pass (the same
     // instructions 12 bytes further on; mesh of 327,680 faces at 1890x536: 23.6 us, aligned
-    // 22.6; 20,480 faces at 1920x1080 with bins of 16 entries, every pair a full bin: 28.1
+    // 22.6; 20,480 faces at 1920x1080 with bins of 16 entries, many of them full: 28.1
     // and 26.0) and changed with any instruction added before it.
     asm volatile(".p2align 6");
     const uint32_t nt = (tx0 <= tx1 && ty0 <= ty1) ? (tx1 - tx0 + 1) * (ty1 - ty0 + 1) : 0u;
